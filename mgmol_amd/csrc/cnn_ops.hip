@@ -34,7 +34,8 @@ namespace
 constexpr int kCh      = 16;
 constexpr int kTaps    = 27;
 constexpr int kWaves   = 4;  // per block
-constexpr int kDwWaves = 1024;
+constexpr int kDwBlocks = 512;  // most blocks of a 16 -> 16 weight gradient: two per CU
+constexpr int kDwPad    = 256;  // bytes after the activations that its last rows read past their end
 
 // parameter offsets (floats)
 constexpr int kW0 = 0, kB0 = kW0 + 27 * 16, kW1 = kB0 + 16, kB1 = kW1 + 27 * 256, kW2 = kB1 + 16,
@@ -472,152 +473,341 @@ __global__ void __launch_bounds__(256) k_conv_out(const uint16_t* __restrict__ h
     out[v] = acc;
 }
 
-// Weight / bias gradient partials of one layer, per wave:
+// The two halves of a dword pair (a in the low half)
+__device__ __forceinline__ uint32_t pack2(uint32_t a, uint32_t b) { return a | (b << 16); }
+
+// Sums a block's four waves' accumulators (in wave order) through LDS and
+// writes them to P: NA fragments D[4g+i][n] at ix(frag, 4g+i, n) of `tot`
+// floats, then the 16 row sums of the last fragment (MFMA against ones).
+template <int NA, class IX>
+__device__ __forceinline__ void dw_block_sum(const f4 (&acc)[NA + 1], float* red, int tot, IX ix, float* __restrict__ P)
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+    for (int w = 0; w < kWaves; w++)
+    {
+        if (wid == w)
+        {
+#pragma unroll
+            for (int k = 0; k < NA; k++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                {
+                    const int q = ix(k, 4 * g + i, n);
+                    if (q >= 0) red[q] = w == 0 ? acc[k][i] : red[q] + acc[k][i];
+                }
+            if (n == 0)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                {
+                    const int q = tot + 4 * g + i;
+                    red[q]      = w == 0 ? acc[NA][i] : red[q] + acc[NA][i];
+                }
+        }
+        __syncthreads();
+    }
+    for (int q = threadIdx.x; q < tot + 16; q += blockDim.x)
+        P[q] = red[q];
+}
+
+// Weight / bias gradient of a 16 -> 16 layer, per block of four waves:
 //   dW[tap][cout][cin] = sum_v dZ[v][cout] H[v + off(tap)][cin],  db = sum_v dZ
-// dZ: BF16 [voxel][16] (COUT = 16) or FP32 scalar (COUT = 1); H: BF16
-// [voxel][16] (CIN = 16) or FP32 scalar (CIN = 1).  A = dZ^T (m = cout,
-// k = voxel), B = H shifted (k = voxel, n = cin, or n = tap for CIN = 1).
-// part[w]: 27*16*16 + 16 floats in the [tap][cout][cin] layout.
-template <int CIN, int COUT>
-__global__ void __launch_bounds__(64) k_conv_dw(const void* __restrict__ dz, const void* __restrict__ hin, int e,
-    int nzt, int64_t nt, float* __restrict__ part)
+// as 16x16x32 MFMAs over voxels: A = dZ^T, B = H.  Each group of 16 lanes
+// (lane n = channel) owns a column (sample, x, 8 z-voxels) and marches along
+// y, so K = 32 is four columns and any box edge fills the lanes.  At row y it
+// holds H[x][y] shifted by dz = -1, 0, 1 (three fragments made from ten 2-byte
+// loads) and the nine dZ rows (x - dx, y - dy) (three new ones per step, the
+// others slide): 27 MFMAs per 34 loads, where one fragment per tap takes
+// four loads each; the next step's loads are in flight during the MFMAs.
+// Bound by those loads, not by the matrix cores.  64 boxes of 32^3: 41 us
+// (0.71 PFLOP/s); one fragment per tap and voxel row took 1744 us.
+// A wave takes the tasks (four columns, one chunk of yl rows) t, t + waves, ...
+template <bool TAIL>
+__global__ void __launch_bounds__(256, 2) k_dw16(const uint16_t* __restrict__ dz, const uint16_t* __restrict__ h,
+    int e, int nzs, int ncol, int yl, int nyc, int ntask, float* __restrict__ part)
 {
-    const int w    = blockIdx.x;
-    const int lane = threadIdx.x, n = lane & 15, g = lane >> 4;
-    constexpr int NACC = CIN == 1 ? 2 : kTaps;
-    f4 acc[NACC];
+    __shared__ float red[kTaps * 256 + 16];
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    f4 acc[kTaps + 1];
 #pragma unroll
-    for (int k = 0; k < NACC; k++)
+    for (int k = 0; k <= kTaps; k++)
         acc[k] = (f4){ 0.f, 0.f, 0.f, 0.f };
-    float bsum = 0.f;
-    for (int64_t t = w; t < nt; t += gridDim.x)
+    const s8 ones = { 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80 };
+    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+    const int64_t rs = (int64_t)e * 16, ps = rs * e;  // row and plane strides
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int t = blockIdx.x * kWaves + wid; t < ntask; t += gridDim.x * kWaves)
     {
-        const TileIx T      = decode(t, e, nzt);
-        const int64_t sbase = (int64_t)T.s * e * e * e;
-        // A: dZ[v = z0 + 4g + i][cout = n]
-        s4 a;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
+        const int cg = t / nyc, y0 = (t - cg * nyc) * yl, y1 = min(e, y0 + yl);
+        const int c  = 4 * cg + g;
+        const bool on = c < ncol;
+        const int cc  = on ? c : 4 * cg;
+        const int zs = cc % nzs, sx = cc / nzs, x = sx % e, z0 = zs * 8;
+        // wave-uniform plane base (one plane before the first column's) and
+        // this lane's 32-bit offsets from it: its own column's plane, channel n
+        // and the ten z-neighbours (the values outside the row are masked)
+        const int sx0          = __builtin_amdgcn_readfirstlane(4 * cg / nzs);
+        const int64_t ubase    = ((int64_t)sx0 - 1) * ps;
+        const uint32_t psb     = 2u * (uint32_t)ps;
+        const uint32_t lane0   = (uint32_t)(sx - sx0 + 1) * psb + 2u * (uint32_t)(z0 * 16 + n);
+        const uint32_t zlo     = z0 > 0 ? 32u : 0u;  // bytes back to z0 - 1
+        // value j (z0 + j - 1) of the row at the wave-uniform address p; a
+        // row's last segment reads on past its end (kDwPad at the end of a buffer)
+        auto at = [&](const char* p, uint32_t o, int j) -> uint32_t {
+            if (j == 0) return *(const uint16_t*)(p + (o - zlo));
+            return *(const uint16_t*)(p + 32 * (j - 1) + o);
+        };
+        const uint32_t mlo = z0 > 0 ? 0xFFFFu : 0u;
+        // position j of the segment is outside the box from j = e - z0 on
+        const int jend = e - z0;
+        uint32_t tm[4] = { ~0u, ~0u, ~0u, ~0u };
+        if (TAIL)
         {
-            const int z = T.z0 + 4 * g + i;
-            float v     = 0.f;
-            if (z < e)
-            {
-                const int64_t vox = sbase + ((int64_t)T.x * e + T.y) * e + z;
-                if (COUT == 16)
-                    v = bf2f(((const uint16_t*)dz)[vox * 16 + n]);
-                else
-                    v = n == 0 ? ((const float*)dz)[vox] : 0.f;
-            }
-            bsum += v;
-            a[i] = (short)f2bf(v);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                tm[k] = (2 * k < jend ? 0xFFFFu : 0u) | (2 * k + 1 < jend ? 0xFFFF0000u : 0u);
         }
-        if (CIN == 16)
-        {
-            const uint16_t* H = (const uint16_t*)hin;
-#pragma unroll 3
-            for (int tap = 0; tap < kTaps; tap++)
-            {
-                s4 b;
-                const int xi = T.x + tap_dx(tap), yi = T.y + tap_dy(tap);
-                const bool rowok = xi >= 0 && xi < e && yi >= 0 && yi < e;
+        const bool xlo = on && x > 0, xhi = on && x < e - 1;
+        // dx = -1, 0, 1: plane x - dx
+        const uint32_t dzo[3] = { lane0 + (xhi ? psb : 0u), lane0, lane0 - (xlo ? psb : 0u) };
+        const bool dzv[3]    = { xhi, on, xlo };
+        uint32_t rh[10], rz[3][8];
+        auto load_h = [&](int y) {
+            const char* p = (const char*)(h + (ubase + (int64_t)y * rs));
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                {
-                    const int z = T.z0 + 4 * g + i, zi = z + tap_dz(tap);
-                    uint16_t v  = 0;
-                    if (rowok && z < e && zi >= 0 && zi < e)
-                        v = H[(sbase + ((int64_t)xi * e + yi) * e + zi) * 16 + n];
-                    b[i] = (short)v;
-                }
-                acc[tap] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[tap], 0, 0, 0);
+            for (int j = 0; j < 10; j++)
+                rh[j] = at(p, lane0, j);
+        };
+        auto load_z = [&](int y) {
+            const char* p = (const char*)(dz + (ubase + (int64_t)min(max(y, 0), e - 1) * rs));
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    rz[d][j] = at(p, dzo[d], j + 1);
+        };
+        s8 a[3][3];  // [dx + 1][row y - 1, y, y + 1]
+        auto pack_z = [&](int y, int row) {
+            const bool yv = y >= 0 && y < e;
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+            {
+                const uint32_t m = yv && dzv[d] ? ~0u : 0u;
+                u4v w;
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    w[k] = pack2(rz[d][2 * k], rz[d][2 * k + 1]) & (TAIL ? m & tm[k] : m);
+                a[d][row] = __builtin_bit_cast(s8, w);
             }
-        }
-        else
+        };
+        load_z(y0 - 1);
+        pack_z(y0 - 1, 0);
+        load_z(y0);
+        pack_z(y0, 1);
+        load_h(y0);
+        load_z(y0 + 1);
+        for (int y = y0; y < y1; y++)
         {
-            const float* X = (const float*)hin;
-#pragma unroll
-            for (int h = 0; h < 2; h++)
+            rh[0] &= mlo;
+            if (TAIL)
             {
-                const int tap = 16 * h + n;
-                s4 b;
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                {
-                    const int z = T.z0 + 4 * g + i;
-                    float v     = 0.f;
-                    if (tap < kTaps && z < e)
+                for (int j = 1; j <= 8; j++)
+                    rh[j + 1] = j >= jend ? 0u : rh[j + 1];
+            }
+            else
+                rh[9] = jend == 8 ? 0u : rh[9];
+            u4v wm, w0, wp;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+            {
+                wm[k] = pack2(rh[2 * k], rh[2 * k + 1]);
+                w0[k] = pack2(rh[2 * k + 1], rh[2 * k + 2]);
+                wp[k] = pack2(rh[2 * k + 2], rh[2 * k + 3]);
+            }
+            const s8 b[3] = { __builtin_bit_cast(s8, wm), __builtin_bit_cast(s8, w0), __builtin_bit_cast(s8, wp) };
+            pack_z(y + 1, 2);
+            if (y + 1 < y1)
+            {
+                load_h(y + 1);
+                load_z(y + 2);
+            }
+#pragma unroll
+            for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+                for (int dy = 0; dy < 3; dy++)  // dZ row y - (dy - 1)
+#pragma unroll
+                    for (int d = 0; d < 3; d++)
                     {
-                        const int xi = T.x + tap_dx(tap), yi = T.y + tap_dy(tap), zi = z + tap_dz(tap);
-                        if (xi >= 0 && xi < e && yi >= 0 && yi < e && zi >= 0 && zi < e)
-                            v = X[sbase + ((int64_t)xi * e + yi) * e + zi];
+                        const int tap = (dx * 3 + dy) * 3 + d;
+                        acc[tap]      = mfma32(a[dx][2 - dy], b[d], acc[tap]);
                     }
-                    b[i] = (short)f2bf(v);
-                }
-                acc[h] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[h], 0, 0, 0);
+            acc[kTaps] = mfma32(a[1][1], ones, acc[kTaps]);
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+            {
+                a[d][0] = a[d][1];
+                a[d][1] = a[d][2];
             }
         }
     }
-    float* P = part + (size_t)w * (kTaps * 256 + 16);
-    // D[m = 4g+i][n]
-    if (CIN == 16)
-    {
-#pragma unroll
-        for (int tap = 0; tap < kTaps; tap++)
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                P[(tap * 16 + 4 * g + i) * 16 + n] = acc[tap][i];
-    }
-    else
-    {
-        // D[cout][tap]: stored at [tap][cout][0]
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-            {
-                const int tap = 16 * h + n;
-                if (tap < kTaps) P[(tap * 16 + 4 * g + i) * 16] = acc[h][i];
-            }
-    }
-    // bias: lanes n, n+16, n+32, n+48 hold cout n's partial sums
-    bsum += __shfl_xor(bsum, 16, 64);
-    bsum += __shfl_xor(bsum, 32, 64);
-    if (g == 0) P[kTaps * 256 + n] = bsum;
+    dw_block_sum<kTaps>(acc, red, kTaps * 256, [](int tap, int co, int ci) { return (tap * 16 + co) * 16 + ci; },
+        part + (size_t)blockIdx.x * (kTaps * 256 + 16));
 }
 
-// sum the per-wave partials in a fixed order into grad[off..] for one layer
-__global__ void k_dw_reduce(const float* part, int nw, int cin, int cout, float* gw, float* gb)
+// Weight gradient of a layer with one scalar side (layer 0: channels dZ0,
+// scalars x; layer 3, FLIP: channels h3, scalars dZ3):
+//   dW[tap][c] = sum_v C[v][c] S[v + off(tap)]   (FLIP: S[v - off(tap)])
+// and the sums of C over v (layer 0's bias), as 16x16x32 MFMAs over voxels,
+// A = C^T, B = S shifted (column = tap, two fragments): 2 MFMAs per 32 voxels
+// where a fragment per tap would use one row or column of 27.  A block marches
+// along x over kSY rows and 32 z-voxels of one sample with the scalars' three
+// planes in an LDS ring as BF16; bound by the 2-byte loads of C.
+// 64 boxes of 32^3: 31 us (layer 0), 28 us (layer 3), where layer 3 with its
+// one output row per tap took 1600 us and layer 0 254 us.
+constexpr int kSY = 8, kSW = kLZ + 4, kSP = (kSY + 2) * kSW;
+template <bool FLIP>
+__global__ void __launch_bounds__(256) k_dw1(const uint16_t* __restrict__ ch, const float* __restrict__ sc, int e,
+    int nyb, int nzb, int nxc, int xl, float* __restrict__ part)
 {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nwq = kTaps * cout * cin;
-    if (q < nwq)
+    __shared__ uint16_t lds[3 * kSP];
+    __shared__ float red[kTaps * 16 + 16];
+    int b        = blockIdx.x;
+    const int xc = b % nxc;
+    b /= nxc;
+    const int zb = b % nzb, yb = (b / nzb) % nyb, s = b / (nzb * nyb);
+    const int x0 = xc * xl, x1 = min(e, x0 + xl), y0 = yb * kSY, z0 = zb * kLZ;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+    const int64_t e3 = (int64_t)e * e * e;
+    const float* S    = sc + (int64_t)s * e3;
+    const uint16_t* C = ch + (int64_t)s * e3 * 16;
+    auto stage = [&](int xp) {
+        uint16_t* dst = lds + ((xp + 3) % 3) * kSP;
+        for (int q = threadIdx.x; q < (kSY + 2) * kLW; q += blockDim.x)
+        {
+            const int yy = q / kLW, zz = q - (q / kLW) * kLW;
+            const int y = y0 - 1 + yy, z = z0 - 1 + zz;
+            float v = 0.f;
+            if (xp >= 0 && xp < e && y >= 0 && y < e && z >= 0 && z < e) v = S[((int64_t)xp * e + y) * e + z];
+            dst[yy * kSW + zz] = f2bf(v);
+        }
+    };
+    // this lane's taps n and 16 + n (the last five columns repeat tap 26 and are dropped)
+    int td[2], to[2];
+#pragma unroll
+    for (int f = 0; f < 2; f++)
     {
-        const int tap = q / (cout * cin), r = q - tap * cout * cin, co = r / cin, ci = r - co * cin;
-        double s = 0.;
-        for (int w = 0; w < nw; w++)
-            s += part[(size_t)w * (kTaps * 256 + 16) + (tap * 16 + co) * 16 + ci];
-        gw[q] = (float)s;
+        const int tap = min(16 * f + n, kTaps - 1), tt = FLIP ? kTaps - 1 - tap : tap;
+        td[f]         = tap_dx(tt);
+        to[f]         = (1 + tap_dy(tt)) * kSW + 1 + tap_dz(tt) + 8 * g;
     }
-    else if (q < nwq + cout)
+    f4 acc[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        acc[k] = (f4){ 0.f, 0.f, 0.f, 0.f };
+    const s8 ones = { 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80 };
+    stage(x0 - 1);
+    stage(x0);
+    for (int x = x0; x < x1; x++)
     {
-        const int co = q - nwq;
-        double s     = 0.;
-        for (int w = 0; w < nw; w++)
-            s += part[(size_t)w * (kTaps * 256 + 16) + kTaps * 256 + co];
-        gb[co] = (float)s;
+        stage(x + 1);
+        // two rows per wave: y0 + wid, y0 + wid + 4; group g: z0 + 8g .. + 7
+        s8 a[2];
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+        {
+            const int y = y0 + wid + 4 * r;
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+            {
+                const int z = z0 + 8 * g + i;
+                a[r][i]     = y < e && z < e ? (short)C[(((int64_t)x * e + y) * e + z) * 16 + n] : (short)0;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+        {
+#pragma unroll
+            for (int f = 0; f < 2; f++)
+            {
+                const uint16_t* row = lds + ((x + 3 + td[f]) % 3) * kSP + (wid + 4 * r) * kSW + to[f];
+                s8 bv;
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    bv[i] = (short)row[i];
+                acc[f] = mfma32(a[r], bv, acc[f]);
+            }
+            acc[2] = mfma32(a[r], ones, acc[2]);
+        }
+        __syncthreads();
+    }
+    dw_block_sum<2>(acc, red, kTaps * 16, [](int f, int c, int k) { return 16 * f + k < kTaps ? (16 * f + k) * 16 + c : -1; },
+        part + (size_t)blockIdx.x * (kTaps * 16 + 16));
+}
+
+// The layers' gradients from their blocks' partials, summed in a fixed order
+// in FP64: a block takes 32 neighbouring values of one layer, eight groups of
+// threads every eighth partial each.  11 us for the four layers of a
+// batch of 64 boxes of 32^3, bound by latency (one thread per value, a chain of
+// 1024 loads: 380 us for each layer).
+struct DwLayer
+{
+    const float* part;
+    float *gw, *gb;
+    int np, nw, nb, stride;  // partials; weights, biases to sum; floats per partial
+};
+struct DwLayers
+{
+    DwLayer l[4];
+    int first[5];  // first block of each layer
+};
+__global__ void __launch_bounds__(256) k_dw_reduce(DwLayers L)
+{
+    __shared__ double red[8][32];
+    int k = 0;
+    while (k < 3 && (int)blockIdx.x >= L.first[k + 1])
+        k++;
+    const DwLayer l = L.l[k];
+    const int col = threadIdx.x & 31, row = threadIdx.x >> 5;
+    const int q = ((int)blockIdx.x - L.first[k]) * 32 + col;
+    double s = 0.;
+    if (q < l.nw + l.nb)
+    {
+        // 16 loads in flight, added in order
+        const float* p = l.part + q;
+        int w          = row;
+        for (; w + 120 < l.np; w += 128)
+        {
+            float v[16];
+#pragma unroll
+            for (int k2 = 0; k2 < 16; k2++)
+                v[k2] = p[(size_t)(w + 8 * k2) * l.stride];
+#pragma unroll
+            for (int k2 = 0; k2 < 16; k2++)
+                s += v[k2];
+        }
+        for (; w < l.np; w += 8)
+            s += p[(size_t)w * l.stride];
+    }
+    red[row][col] = s;
+    __syncthreads();
+    if (row == 0 && q < l.nw + l.nb)
+    {
+        for (int r = 1; r < 8; r++)
+            s += red[r][col];
+        (q < l.nw ? l.gw[q] : l.gb[q - l.nw]) = (float)s;
     }
 }
 
-// loss pieces: y = s x + z; d = y - t; dy = 2 d / N; per block sums of d^2
-// and dy*x (for ds), written to part[2*block]
+// loss pieces: y = s x + z; d = y - t; dy = 2 d / N; per block sums of d^2,
+// dy*x (for ds) and dy (layer 3's bias), written to part[3*block]
 __global__ void __launch_bounds__(256) k_loss(const float* x, const float* z, const float* t, const float* prm,
     int64_t n, float* y, float* dy, double* part)
 {
-    __shared__ double red[2][4];
+    __shared__ double red[3][4];
     const float s   = prm[kS];
     const double sc = 2.0 / (double)n;
-    double a = 0., b = 0.;
+    double a = 0., b = 0., c = 0.;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     {
         const float yv = s * x[i] + z[i];
@@ -629,24 +819,47 @@ __global__ void __launch_bounds__(256) k_loss(const float* x, const float* z, co
             dy[i]          = g;
             a += d * d;
             b += (double)g * (double)x[i];
+            c += (double)g;
         }
     }
     for (int o = 32; o > 0; o >>= 1)
     {
         a += __shfl_xor(a, o, 64);
         b += __shfl_xor(b, o, 64);
+        c += __shfl_xor(c, o, 64);
     }
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (lane == 0)
     {
         red[0][wid] = a;
         red[1][wid] = b;
+        red[2][wid] = c;
     }
     __syncthreads();
-    if (threadIdx.x == 0)
+    if (threadIdx.x < 3)
     {
-        part[2 * blockIdx.x]     = red[0][0] + red[0][1] + red[0][2] + red[0][3];
-        part[2 * blockIdx.x + 1] = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+        const double* r                   = red[threadIdx.x];
+        part[3 * blockIdx.x + threadIdx.x] = r[0] + r[1] + r[2] + r[3];
+    }
+}
+
+// the loss blocks' sums: ds and layer 3's bias gradient to the gradient, the
+// sum of d^2 to loss
+__global__ void __launch_bounds__(192) k_loss_sum(const double* part, int np, float* grad, double* loss)
+{
+    // wave q sums column q, lane l every 64th block
+    const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    double s = 0.;
+    for (int k = lane; k < np; k += 64)
+        s += part[3 * k + q];
+    for (int o = 32; o > 0; o >>= 1)
+        s += __shfl_xor(s, o, 64);
+    if (lane == 0)
+    {
+        if (q == 0)
+            *loss = s;
+        else
+            grad[q == 1 ? kS : kB3] = (float)s;
     }
 }
 
@@ -744,7 +957,8 @@ struct mgx_cnn
     uint16_t *f0, *f1, *f2, *f3, *r3, *r2, *r1;
     // activations for max_batch samples
     uint16_t *h1 = nullptr, *h2 = nullptr, *h3 = nullptr, *dza = nullptr, *dzb = nullptr;
-    float *z = nullptr, *y = nullptr, *dy = nullptr, *xf = nullptr, *part = nullptr;
+    float *z = nullptr, *y = nullptr, *dy = nullptr, *xf = nullptr;
+    float *part0 = nullptr, *part1 = nullptr, *part2 = nullptr, *part3 = nullptr;  // weight-gradient partials per layer
     double *lpart = nullptr, *rms = nullptr;
     double* host  = nullptr;  // pinned
     bool dirty    = true;     // BF16 weights need refreshing
@@ -756,6 +970,21 @@ namespace
 {
 
 constexpr int kLossBlocks = 1024;
+
+// planes per x-chunk of a scalar layer's weight gradient: the columns alone
+// when they give four blocks per CU, else chunks of at least four planes
+int dw1_xl(int e, int64_t cols)
+{
+    const int64_t want = std::max<int64_t>(1, std::min<int64_t>(1024 / cols, (e + 3) / 4));
+    return (int)((e + want - 1) / want);
+}
+
+// most blocks of dw1 over batches of 1..max_batch samples
+int64_t dw1_blocks(int e, int max_batch)
+{
+    const int64_t per = (int64_t)((e + kSY - 1) / kSY) * ((e + kLZ - 1) / kLZ);
+    return std::max<int64_t>(1024 + per, per * max_batch);
+}
 
 int64_t ntiles(int e, int nb) { return (int64_t)nb * e * e * ((e + 15) / 16); }
 
@@ -804,18 +1033,34 @@ int forward(mgx_cnn* c, const float* x, int nb)
     return forward_any<float>(c, x, nullptr, nullptr, nb, nullptr);
 }
 
-template <int CIN, int COUT>
-int dw(mgx_cnn* c, const void* dz, const void* hin, int nb, int woff, int boff, int cin, int cout)
+// The launch of a weight gradient: 16 -> 16 layers in at most kDwBlocks blocks
+// (two resident per CU), with chunks of rows only where the columns alone
+// leave waves idle; scalar layers one block per (8 rows, 32 z, x-chunk).
+int dw16(mgx_cnn* c, const uint16_t* dz, const uint16_t* h, int nb, float* part, DwLayer& l)
 {
-    mgx_ctx* ctx     = c->ctx;
-    const int e      = c->edge, nzt = (e + 15) / 16;
-    const int64_t nt = ntiles(e, nb);
-    const int nw     = (int)std::min<int64_t>(kDwWaves, nt);
-    hipLaunchKernelGGL((k_conv_dw<CIN, COUT>), dim3(nw), dim3(64), 0, ctx->stream, dz, hin, e, nzt, nt, c->part);
-    const int nq = kTaps * cin * cout + cout;
-    hipLaunchKernelGGL(k_dw_reduce, dim3((nq + 255) / 256), dim3(256), 0, ctx->stream, (const float*)c->part, nw,
-        cin, cout, c->g + woff, c->g + boff);
+    mgx_ctx* ctx  = c->ctx;
+    const int e   = c->edge, nzs = (e + 7) / 8, ncol = nb * e * nzs, ncg = (ncol + 3) / 4;
+    const int want = std::max(1, std::min(kDwBlocks * kWaves / ncg, (e + 3) / 4));
+    const int yl = (e + want - 1) / want, nyc = (e + yl - 1) / yl;
+    const int ntask = ncg * nyc, blocks = std::min(kDwBlocks, (ntask + kWaves - 1) / kWaves);
+    if (e % 8)
+        hipLaunchKernelGGL(k_dw16<true>, dim3(blocks), dim3(256), 0, ctx->stream, dz, h, e, nzs, ncol, yl, nyc, ntask, part);
+    else
+        hipLaunchKernelGGL(k_dw16<false>, dim3(blocks), dim3(256), 0, ctx->stream, dz, h, e, nzs, ncol, yl, nyc, ntask, part);
     MGX_CHECK_LAUNCH(ctx);
+    l.part = part, l.np = blocks, l.nw = kTaps * 256, l.nb = 16, l.stride = kTaps * 256 + 16;
+    return MGX_OK;
+}
+
+template <bool FLIP>
+int dw1(mgx_cnn* c, const uint16_t* ch, const float* sc, int nb, float* part, DwLayer& l)
+{
+    mgx_ctx* ctx  = c->ctx;
+    const int e   = c->edge, nyb = (e + kSY - 1) / kSY, nzb = (e + kLZ - 1) / kLZ, cols = nb * nyb * nzb;
+    const int xl  = dw1_xl(e, cols), nxc = (e + xl - 1) / xl;
+    hipLaunchKernelGGL(k_dw1<FLIP>, dim3(cols * nxc), dim3(256), 0, ctx->stream, ch, sc, e, nyb, nzb, nxc, xl, part);
+    MGX_CHECK_LAUNCH(ctx);
+    l.part = part, l.np = cols * nxc, l.nw = kTaps * 16, l.nb = FLIP ? 0 : 16, l.stride = kTaps * 16 + 16;
     return MGX_OK;
 }
 
@@ -830,41 +1075,43 @@ int grad(mgx_cnn* c, const float* x, const float* t, int nb, double* loss)
     const int64_t nt = ntiles(e, nb);
     hipLaunchKernelGGL(k_loss, dim3(kLossBlocks), dim3(256), 0, ctx->stream, x, (const float*)c->z, t,
         (const float*)c->p, n, (float*)nullptr, c->dy, c->lpart);
+    hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(192), 0, ctx->stream, (const double*)c->lpart, kLossBlocks, c->g,
+        c->lpart + 3 * kLossBlocks);
     MGX_CHECK_LAUNCH(ctx);
-    // layer 3: dZ3 = dy (scalar)
-    if ((rc = dw<16, 1>(c, c->dy, c->h3, nb, kW3, kB3, 16, 1))) return rc;
+    DwLayers L;
+    // layer 3: dZ3 = dy (scalar; its bias came with the loss)
+    if ((rc = dw1<true>(c, c->h3, c->dy, nb, c->part3, L.l[3]))) return rc;
+    L.l[3].gw = c->g + kW3, L.l[3].gb = nullptr;
     const dim3 grid((unsigned)((nt + kWaves - 1) / kWaves)), blk(64 * kWaves);
     hipLaunchKernelGGL((k_conv<1, 16, CONV_BWD_MASK>), grid, blk, 0, ctx->stream, (const void*)c->dy, c->r3,
         (const float*)nullptr, (void*)c->dza, (const uint16_t*)c->h3, e, nzt, nt);
     MGX_CHECK_LAUNCH(ctx);
     // layer 2: dZ2 = dza
-    if ((rc = dw<16, 16>(c, c->dza, c->h2, nb, kW2, kB2, 16, 16))) return rc;
+    if ((rc = dw16(c, c->dza, c->h2, nb, c->part2, L.l[2]))) return rc;
+    L.l[2].gw = c->g + kW2, L.l[2].gb = c->g + kB2;
     const int nyb = (e + kLY - 1) / kLY, nzb = (e + kLZ - 1) / kLZ;
     const dim3 lgrid((unsigned)(nb * nyb * nzb));
     hipLaunchKernelGGL((k_conv16_lds<CONV_BWD_MASK>), lgrid, dim3(256), 0, ctx->stream, (const uint16_t*)c->dza,
         (const uint16_t*)c->r2, (const float*)nullptr, c->dzb, (const uint16_t*)c->h2, e, nyb, nzb);
     MGX_CHECK_LAUNCH(ctx);
     // layer 1: dZ1 = dzb
-    if ((rc = dw<16, 16>(c, c->dzb, c->h1, nb, kW1, kB1, 16, 16))) return rc;
+    if ((rc = dw16(c, c->dzb, c->h1, nb, c->part1, L.l[1]))) return rc;
+    L.l[1].gw = c->g + kW1, L.l[1].gb = c->g + kB1;
     hipLaunchKernelGGL((k_conv16_lds<CONV_BWD_MASK>), lgrid, dim3(256), 0, ctx->stream, (const uint16_t*)c->dzb,
         (const uint16_t*)c->r1, (const float*)nullptr, c->dza, (const uint16_t*)c->h1, e, nyb, nzb);
     MGX_CHECK_LAUNCH(ctx);
     // layer 0: dZ0 = dza, input x
-    if ((rc = dw<1, 16>(c, c->dza, x, nb, kW0, kB0, 1, 16))) return rc;
-    // loss and ds
-    MGX_CHECK_HIP(ctx, hipMemcpyAsync(c->host, c->lpart, 2 * kLossBlocks * sizeof(double), hipMemcpyDeviceToHost,
+    if ((rc = dw1<false>(c, c->dza, x, nb, c->part0, L.l[0]))) return rc;
+    L.l[0].gw = c->g + kW0, L.l[0].gb = c->g + kB0;
+    L.first[0] = 0;
+    for (int k = 0; k < 4; k++)
+        L.first[k + 1] = L.first[k] + (L.l[k].nw + L.l[k].nb + 31) / 32;
+    hipLaunchKernelGGL(k_dw_reduce, dim3(L.first[4]), dim3(256), 0, ctx->stream, L);
+    MGX_CHECK_LAUNCH(ctx);
+    MGX_CHECK_HIP(ctx, hipMemcpyAsync(c->host, c->lpart + 3 * kLossBlocks, sizeof(double), hipMemcpyDeviceToHost,
                            ctx->stream));
     MGX_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    double a = 0., b = 0.;
-    for (int k = 0; k < kLossBlocks; k++)
-    {
-        a += c->host[2 * k];
-        b += c->host[2 * k + 1];
-    }
-    const float ds = (float)b;
-    MGX_CHECK_HIP(ctx, hipMemcpyAsync(c->g + kS, &ds, sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-    MGX_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    *loss = a / (double)n;
+    *loss = c->host[0] / (double)n;
     return MGX_OK;
 }
 
@@ -890,7 +1137,7 @@ int mgx_cnn_create(mgx_ctx* ctx, int edge, int max_batch, mgx_cnn** out)
     c->edge      = edge;
     c->max_batch = max_batch;
     const size_t nv = (size_t)max_batch * edge * edge * edge;
-    const int nw    = kDwWaves;
+    const size_t nd16 = (size_t)kDwBlocks * (kTaps * 256 + 16), nd1 = (size_t)dw1_blocks(edge, max_batch) * (kTaps * 16 + 16);
     bool ok         = true;
     auto al         = [&](void** p, size_t bytes) { ok = ok && hipMalloc(p, std::max<size_t>(bytes, 256)) == hipSuccess; };
     al((void**)&c->p, kNP * sizeof(float));
@@ -898,19 +1145,22 @@ int mgx_cnn_create(mgx_ctx* ctx, int edge, int max_batch, mgx_cnn** out)
     al((void**)&c->m, kNP * sizeof(float));
     al((void**)&c->v, kNP * sizeof(float));
     al((void**)&c->wbf, (2 * 512 + 5 * kTaps * 256) * sizeof(uint16_t));
-    al((void**)&c->h1, nv * 16 * sizeof(uint16_t));
-    al((void**)&c->h2, nv * 16 * sizeof(uint16_t));
-    al((void**)&c->h3, nv * 16 * sizeof(uint16_t));
-    al((void**)&c->dza, nv * 16 * sizeof(uint16_t));
-    al((void**)&c->dzb, nv * 16 * sizeof(uint16_t));
+    al((void**)&c->h1, nv * 16 * sizeof(uint16_t) + kDwPad);
+    al((void**)&c->h2, nv * 16 * sizeof(uint16_t) + kDwPad);
+    al((void**)&c->h3, nv * 16 * sizeof(uint16_t) + kDwPad);
+    al((void**)&c->dza, nv * 16 * sizeof(uint16_t) + kDwPad);
+    al((void**)&c->dzb, nv * 16 * sizeof(uint16_t) + kDwPad);
     al((void**)&c->z, nv * sizeof(float));
     al((void**)&c->y, nv * sizeof(float));
     al((void**)&c->dy, nv * sizeof(float));
     al((void**)&c->xf, nv * sizeof(float));
-    al((void**)&c->part, (size_t)nw * (kTaps * 256 + 16) * sizeof(float));
-    al((void**)&c->lpart, 2 * kLossBlocks * sizeof(double));
+    al((void**)&c->part0, nd1 * sizeof(float));
+    al((void**)&c->part1, nd16 * sizeof(float));
+    al((void**)&c->part2, nd16 * sizeof(float));
+    al((void**)&c->part3, nd1 * sizeof(float));
+    al((void**)&c->lpart, (3 * kLossBlocks + 1) * sizeof(double));
     al((void**)&c->rms, (size_t)max_batch * sizeof(double));
-    ok = ok && hipHostMalloc((void**)&c->host, 2 * kLossBlocks * sizeof(double), hipHostMallocDefault) == hipSuccess;
+    ok = ok && hipHostMalloc((void**)&c->host, sizeof(double), hipHostMallocDefault) == hipSuccess;
     if (!ok)
     {
         mgx_cnn_destroy(c);
@@ -939,7 +1189,7 @@ int mgx_cnn_destroy(mgx_cnn* c)
 {
     if (!c) return MGX_OK;
     void* bufs[] = { c->p, c->g, c->m, c->v, c->wbf, c->h1, c->h2, c->h3, c->dza, c->dzb, c->z, c->y, c->dy, c->xf,
-        c->part, c->lpart, c->rms };
+        c->part0, c->part1, c->part2, c->part3, c->lpart, c->rms };
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (c->host) (void)hipHostFree(c->host);

@@ -67,6 +67,34 @@ def test_cnn_grad_matches_oracle(ctx):
     net.close()
 
 
+@pytest.mark.parametrize("edge,nb", [(1, 3), (5, 4), (8, 1), (9, 2), (20, 2), (33, 1), (40, 1)])
+def test_cnn_grad_edges(ctx, edge, nb):
+    """The weight gradients take eight z-voxels a lane group, four columns a
+    wave and chunks of rows: one segment, ragged last segments, rows and
+    columns that do not fill a block, one sample and a few.  The oracle rounds
+    weights and activations to BF16 at the same points; what is left are FP32
+    sums in another order and the activations (2^-9 each) that they move across
+    a rounding boundary, under 3e-2 of a tensor as in the test above.  A wrong
+    tap, column or mask is an error of order one."""
+    p = _params(5)
+    rng = np.random.default_rng(edge)
+    x = rng.standard_normal((nb, edge, edge, edge)).astype(np.float32)
+    t = (0.5 * x + 0.1 * rng.standard_normal(x.shape)).astype(np.float32)
+    net = learned.Cnn(ctx, edge, nb + 1, p)
+    tx, tt = to_dev(x), to_dev(t)
+    loss, g = net.grad(tx, tt, nb)
+    Lr, gr = OC.backward(p, x, t, bf16_mode=True)
+    assert loss == pytest.approx(Lr, rel=2e-3)
+    for name in learned.NAMES:
+        err = _rel(g[name], gr[name])
+        say("grad", edge, nb, name, err)
+        assert err < 3e-2, name
+    # the same bits from a second call on the same network
+    again = net.grad(tx, tt, nb)
+    assert again[0] == loss and all(np.array_equal(again[1][k], g[k]) for k in learned.NAMES)
+    net.close()
+
+
 def test_cnn_training_reduces_loss(ctx):
     """Adam on a smoothing target (t = local 3^3 average of x): the loss falls
     well below the untrained network's."""

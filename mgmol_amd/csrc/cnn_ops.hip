@@ -14,16 +14,15 @@
 //   w3[27][1][16] b3[1] s
 // with tap = (dx*3 + dy)*3 + dz for the offset (dx-1, dy-1, dz-1).
 //
-// Convolution as MFMA (v_mfma_f32_16x16x16_bf16): one wave computes a tile
-// of 16 z-consecutive voxels x 16 output channels, D[cout][voxel] =
-// sum_tap W_tap[cout][cin] X[cin][voxel + off(tap)]: A = weights (held in
-// registers for all taps), B = input rows (8-byte loads, 16 voxels x 32 B
-// contiguous per tap).  Lane l holds A[l%16][4(l/16)+i], B[4(l/16)+i][l%16]
-// and D[4(l/16)+i][l%16].
+// Convolution as MFMA (v_mfma_f32_16x16x32_bf16): a tile is 16 z-consecutive
+// voxels x 16 output channels, D[cout][voxel] = sum_tap W_tap[cout][cin]
+// X[cin][voxel + off(tap)], with the weights of all taps in registers and the
+// input rows in LDS, two taps of 16 channels per MFMA.
 #include "common.hpp"
 
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 namespace mgx
@@ -75,402 +74,384 @@ __device__ inline int tap_dx(int t) { return t / 9 - 1; }
 __device__ inline int tap_dy(int t) { return (t / 3) % 3 - 1; }
 __device__ inline int tap_dz(int t) { return t % 3 - 1; }
 
-struct TileIx
-{
-    int s, x, y, z0;
-};
-
-__device__ inline TileIx decode(int64_t t, int e, int nzt)
-{
-    TileIx r;
-    const int64_t per = (int64_t)e * e * nzt;
-    r.s               = (int)(t / per);
-    int64_t q         = t - (int64_t)r.s * per;
-    r.x               = (int)(q / ((int64_t)e * nzt));
-    q -= (int64_t)r.x * e * nzt;
-    r.y  = (int)(q / nzt);
-    r.z0 = (int)(q - (int64_t)r.y * nzt) * 16;
-    return r;
-}
-
 enum
 {
-    CONV_FWD_RELU = 0,  // + bias, ReLU, BF16 out
-    CONV_FWD_LIN  = 1,  // + bias, FP32 out (last layer)
-    CONV_BWD_MASK = 2   // no bias, times (hmask > 0), BF16 out
+    CONV_FWD_RELU = 0,  // + bias, ReLU
+    CONV_BWD_MASK = 1   // no bias, times (hmask > 0)
 };
 
-// One conv layer over nt tiles.  CIN = 1: input FP32 scalar per voxel,
-// weights [16 cout][32 taps] BF16 (taps >= 27 zero).  CIN = 16: input BF16
-// [voxel][16], weights [27][16 cout][16 cin] BF16.  COUT = 16: output
-// [voxel][16]; COUT = 1: FP32 scalar (row 0 of D; weights rows 1..15 zero).
-template <int CIN, int COUT, int MODE>
-__global__ void __launch_bounds__(64 * kWaves) k_conv(const void* __restrict__ in, const uint16_t* __restrict__ wt,
-    const float* __restrict__ bias, void* __restrict__ out, const uint16_t* __restrict__ hmask, int e, int nzt,
-    int64_t nt)
+// value pairs to BF16 (nearest even; v_cvt_pk_bf16_f32), the first in the low half
+__device__ __forceinline__ uint32_t cvt2(float a, float b)
 {
-    const int64_t t = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6);
-    if (t >= nt) return;  // whole wave
-    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
-    const TileIx T = decode(t, e, nzt);
-    const int64_t sbase = (int64_t)T.s * e * e * e;
-    f4 acc = { 0.f, 0.f, 0.f, 0.f };
-    if (CIN == 16)
-    {
-        // all 27 input loads in flight before the MFMA chain
-        const uint16_t* X = (const uint16_t*)in;
-        s4 b[kTaps];
-#pragma unroll
-        for (int tap = 0; tap < kTaps; tap++)
-        {
-            const int xi = T.x + tap_dx(tap), yi = T.y + tap_dy(tap), zi = T.z0 + n + tap_dz(tap);
-            b[tap] = (s4){ 0, 0, 0, 0 };
-            if (xi >= 0 && xi < e && yi >= 0 && yi < e && zi >= 0 && zi < e)
-                b[tap] = *(const s4*)(X + (sbase + ((int64_t)xi * e + yi) * e + zi) * 16 + 4 * g);
-        }
-#pragma unroll
-        for (int tap = 0; tap < kTaps; tap++)
-        {
-            const s4 a = *(const s4*)(wt + ((size_t)tap * 16 + n) * 16 + 4 * g);
-            acc        = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[tap], acc, 0, 0, 0);
-        }
-    }
-    else
-    {
-        const float* X = (const float*)in;
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-        {
-            const s4 a = *(const s4*)(wt + (size_t)n * 32 + 16 * h + 4 * g);
-            s4 b;
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-            {
-                const int tap = 16 * h + 4 * g + i;
-                float v       = 0.f;
-                if (tap < kTaps)
-                {
-                    const int xi = T.x + tap_dx(tap), yi = T.y + tap_dy(tap), zi = T.z0 + n + tap_dz(tap);
-                    if (xi >= 0 && xi < e && yi >= 0 && yi < e && zi >= 0 && zi < e)
-                        v = X[sbase + ((int64_t)xi * e + yi) * e + zi];
-                }
-                b[i] = (short)f2bf(v);
-            }
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-        }
-    }
-    const int z = T.z0 + n;
-    if (z >= e) return;
-    const int64_t vox = sbase + ((int64_t)T.x * e + T.y) * e + z;
-    if (COUT == 1)
-    {
-        if (g == 0) ((float*)out)[vox] = acc[0] + (MODE == CONV_BWD_MASK ? 0.f : bias[0]);
-        return;
-    }
-    s4 o;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-    {
-        float v = acc[i];
-        if (MODE == CONV_FWD_RELU) v = fmaxf(v + bias[4 * g + i], 0.f);
-        if (MODE == CONV_FWD_LIN) v += bias[4 * g + i];
-        if (MODE == CONV_BWD_MASK && hmask[vox * 16 + 4 * g + i] == 0) v = 0.f;
-        o[i] = (short)f2bf(v);
-    }
-    *(s4*)((uint16_t*)out + vox * 16 + 4 * g) = o;
+    bf2 v;
+    v[0] = (__bf16)a;
+    v[1] = (__bf16)b;
+    return __builtin_bit_cast(uint32_t, v);
 }
 
-// A 16 -> 16 layer with the input staged in LDS: a block (4 waves) owns
-// rows y0..y0+3 and z0..z0+31 of one sample and marches along x, keeping the
-// planes x-1, x, x+1 of its (6 x 34)-voxel window in a ring of 3 LDS slots
-// (one new plane loaded per step, 16-byte coalesced loads, zeros outside the
-// box).  Wave w computes row y0+w, two 16-voxel z-tiles, 27 MFMAs each, with
-// all 27 taps' weights in registers and the B operands read from LDS.
-constexpr int kLY = 4, kLZ = 32, kLW = kLZ + 2, kLH = kLY + 2;
-constexpr int kPlane = kLH * kLW * 16;  // BF16 values per staged plane
-
-template <int MODE>
-__global__ void __launch_bounds__(256) k_conv16_lds(const uint16_t* __restrict__ in, const uint16_t* __restrict__ wt,
-    const float* __restrict__ bias, uint16_t* __restrict__ out, const uint16_t* __restrict__ hmask, int e, int nyb,
-    int nzb)
+// A 16-channel layer's input window of ROWS x 34 voxels (one plane of x) in
+// LDS, the two 8-channel halves apart, so that 16 lanes reading neighbouring
+// voxels touch 256 contiguous bytes.  Every thread keeps its chunks' places:
+// load() puts the next plane in registers, store() moves it to LDS.
+constexpr int kLZ = 32, kLW = kLZ + 2;
+template <int ROWS>
+struct Window
 {
-    __shared__ __align__(16) uint16_t lds[3 * kPlane];
-    const int b = blockIdx.x;
-    const int s = b / (nyb * nzb), yb = (b / nzb) % nyb, zb = b % nzb;
-    const int y0 = yb * kLY, z0 = zb * kLZ;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
-    const int64_t e3 = (int64_t)e * e * e;
-    const uint16_t* X = in + (int64_t)s * e3 * 16;
-    // K = 32 per MFMA: tap pair tp, lane group g: tap 2tp + (g >> 1), channels
-    // 8(g & 1)..8(g & 1)+7 (the 28th tap is zero)
-    constexpr int kPairs = (kTaps + 1) / 2;
-    const int tsel = g >> 1, cs = 8 * (g & 1);
-    s8 wa[kPairs];
-#pragma unroll
-    for (int tp = 0; tp < kPairs; tp++)
+    static constexpr int kHalf = ROWS * kLW * 8;  // BF16 values per half
+    static constexpr int kSize = 2 * kHalf;
+    static constexpr int kN    = (ROWS * kLW * 2 + 255) / 256;
+    const uint16_t* X;
+    int64_t plane;
+    int e, off[kN], dst[kN];
+    uint4 v[kN];
+    __device__ __forceinline__ Window(const uint16_t* x, int e_, int y0, int z0) : X(x), e(e_)
     {
-        const int tap = 2 * tp + tsel;
-        wa[tp]        = tap < kTaps ? *(const s8*)(wt + ((size_t)tap * 16 + n) * 16 + cs) : (s8){ 0, 0, 0, 0, 0, 0, 0, 0 };
-    }
-    // stage plane xp into slot, as 16-byte chunks (2 per voxel)
-    auto stage = [&](int xp, int slot) {
-        uint4* dst = (uint4*)(lds + slot * kPlane);
-        for (int q = threadIdx.x; q < kLH * kLW * 2; q += blockDim.x)
+        plane = (int64_t)e * e * 16;
+#pragma unroll
+        for (int k = 0; k < kN; k++)
         {
-            const int vox = q >> 1, half = q & 1;
-            const int yy = vox / kLW, zz = vox - (vox / kLW) * kLW;
-            const int y = y0 - 1 + yy, z = z0 - 1 + zz;
-            uint4 v = { 0u, 0u, 0u, 0u };
-            if (xp >= 0 && xp < e && y >= 0 && y < e && z >= 0 && z < e)
-                v = *(const uint4*)(X + (((int64_t)xp * e + y) * e + z) * 16 + 8 * half);
-            dst[q] = v;
+            const int q = threadIdx.x + 256 * k, half = q & 1, vox = q >> 1, yy = vox / kLW;
+            const int y = y0 - 1 + yy, z = z0 - 1 + vox - yy * kLW;
+            const bool in = q < ROWS * kLW * 2;
+            off[k] = in && y >= 0 && y < e && z >= 0 && z < e ? (y * e + z) * 16 + 8 * half : -1;
+            dst[k] = in ? half * kHalf + vox * 8 : -1;
+        }
+    }
+    __device__ __forceinline__ void load(int xp)
+    {
+#pragma unroll
+        for (int k = 0; k < kN; k++)
+        {
+            v[k] = (uint4){ 0u, 0u, 0u, 0u };
+            if (off[k] >= 0 && xp < e) v[k] = *(const uint4*)(X + xp * plane + off[k]);
+        }
+    }
+    __device__ __forceinline__ void store(uint16_t* lds) const
+    {
+#pragma unroll
+        for (int k = 0; k < kN; k++)
+            if (dst[k] >= 0) *(uint4*)(lds + dst[k]) = v[k];
+    }
+};
+
+// A 16 -> 16 layer.  A block (4 waves) owns rows y0..y0+3, z0..z0+31 of one
+// sample and marches along x; wave w computes row y0+w, two 16-voxel z-tiles,
+// as D[cout][voxel] += W_tap[cout][cin] X[cin][voxel + off(tap)] with
+// 16x16x32 MFMAs (K = two taps of 16 channels).  Each plane of the input is
+// in LDS once (two buffers, one barrier per plane, the next plane's loads in
+// flight) and enters the three planes of output it reaches (dx = 1, 0, -1),
+// whose sums stay in registers: five operand reads per 15 MFMAs, where a
+// three-plane ring with one output plane reads 14 per 14.  Taps in pairs:
+// (dz = -1, 0) of a row, then dz = 1 of rows y-1, y and of row y+1 (against
+// zero weights in its second half).
+// Bound by the planes' load latency between the matrix and the memory limits.
+// 256 boxes of 32^3 (537 MB, 116 GFLOP): 157 us (3.4 TB/s, 0.74 PFLOP/s); the
+// three-plane ring took 240 us.
+constexpr int kLY = 4, kLH = kLY + 2;
+template <int MODE>
+__global__ void __launch_bounds__(256, 4) k_conv16(const uint16_t* __restrict__ in, const uint16_t* __restrict__ wt,
+    const float* __restrict__ bias, uint16_t* __restrict__ out, const uint16_t* __restrict__ hmask, int e, int nyb,
+    int nzb, int nxc, int xl)
+{
+    typedef Window<kLH> W;
+    __shared__ __align__(16) uint16_t lds[2][W::kSize];
+    int b        = blockIdx.x;
+    const int xc = b % nxc;
+    b /= nxc;
+    const int s = b / (nyb * nzb), y0 = (b / nzb) % nyb * kLY, z0 = b % nzb * kLZ;
+    const int x0 = xc * xl, x1 = min(e, x0 + xl);
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+    const int tsel = g >> 1, cs = 8 * (g & 1);
+    const int64_t e3 = (int64_t)e * e * e;
+    s8 wa[3][5];  // [dx + 1][pair]
+#pragma unroll
+    for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+        for (int k = 0; k < 5; k++)
+        {
+            const int tap = k < 3 ? (dx * 3 + k) * 3 + tsel : (dx * 3 + (k == 3 ? tsel : 2)) * 3 + 2;
+            wa[dx][k]     = *(const s8*)(wt + ((size_t)tap * 16 + n) * 16 + cs);
+            if (k == 4 && tsel) wa[dx][k] = (s8){ 0, 0, 0, 0, 0, 0, 0, 0 };
+        }
+    f4 bv = { 0.f, 0.f, 0.f, 0.f };
+    if (MODE == CONV_FWD_RELU) bv = *(const f4*)(bias + 4 * g);
+    // the pairs' places in the window: rows wid, wid+1, wid+2 (= y-1, y, y+1)
+    const int hb = (g & 1) * W::kHalf, p0 = hb + (wid * kLW + n + tsel) * 8;
+    const int q0 = hb + ((wid + tsel) * kLW + n + 2) * 8, q1 = hb + ((wid + 2) * kLW + n + 2) * 8;
+    const int y = y0 + wid;
+    W w(in + (int64_t)s * e3 * 16, e, y0, z0);
+    // this lane's outputs: voxels z0 + n (+ 16) of its row, channels 4g..4g+3
+    const int64_t vox0 = ((int64_t)s * e3 + (int64_t)y * e + z0 + n) * 16 + 4 * g, e2 = (int64_t)e * e * 16;
+    const bool ok[2]   = { y < e && z0 + n < e, y < e && z0 + 16 + n < e };
+    uint2 mp[2], mc[2];  // the masks of planes xp - 1, xp: loaded a plane ahead of their use
+    auto emit = [&](int x, const f4 (&a)[2], const uint2 (&mask)[2]) {
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+        {
+            if (!ok[t]) continue;
+            float v[4];
+            if (MODE == CONV_BWD_MASK)
+            {
+                const uint2 m = mask[t];
+                v[0] = m.x & 0xFFFFu ? a[t][0] : 0.f;
+                v[1] = m.x >> 16 ? a[t][1] : 0.f;
+                v[2] = m.y & 0xFFFFu ? a[t][2] : 0.f;
+                v[3] = m.y >> 16 ? a[t][3] : 0.f;
+            }
+            else
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    v[i] = fmaxf(a[t][i] + bv[i], 0.f);
+            *(uint2*)(out + vox0 + x * e2 + 256 * t) = (uint2){ cvt2(v[0], v[1]), cvt2(v[2], v[3]) };
         }
     };
-    stage(-1, 2);  // zeros
-    stage(0, 0);
-    const int y = y0 + wid;
-    for (int x = 0; x < e; x++)
+    const f4 zero = { 0.f, 0.f, 0.f, 0.f };
+    const bool two = z0 + 16 < e;  // the second z-tile holds voxels
+    f4 c0[2] = { zero, zero }, c1[2] = { zero, zero }, c2[2] = { zero, zero };  // sums of planes xp + 1, xp, xp - 1
+    const int xa = max(x0 - 1, 0), xb = min(x1, e - 1);
+    w.load(xa);
+    for (int xp = xa; xp <= xb; xp++)
     {
-        stage(x + 1, (x + 1) % 3);
+        uint16_t* buf = lds[xp & 1];
+        w.store(buf);
         __syncthreads();
-        f4 acc0 = { 0.f, 0.f, 0.f, 0.f }, acc1 = acc0;
-#pragma unroll
-        for (int tp = 0; tp < kPairs; tp++)
-        {
-            // the padding tap (27) reads tap 26's operands against zero weights
-            const int tap  = min(2 * tp + tsel, kTaps - 1);
-            const int slot = (x + 3 + tap_dx(tap)) % 3;
-            const int yy   = wid + 1 + tap_dy(tap);
-            const uint16_t* row = lds + slot * kPlane + (yy * kLW) * 16;
-            const int zz = n + 1 + tap_dz(tap);
-            const s8 b0 = *(const s8*)(row + zz * 16 + cs);
-            const s8 b1 = *(const s8*)(row + (zz + 16) * 16 + cs);
-            acc0 = mfma32(wa[tp], b0, acc0);
-            acc1 = mfma32(wa[tp], b1, acc1);
-        }
-        if (y < e)
-        {
+        if (MODE == CONV_BWD_MASK)
 #pragma unroll
             for (int t = 0; t < 2; t++)
             {
-                const int z = z0 + 16 * t + n;
-                if (z >= e) continue;
-                const int64_t vox = (int64_t)s * e3 + ((int64_t)x * e + y) * e + z;
-                const f4 a = t == 0 ? acc0 : acc1;
-                s4 o;
+                mp[t] = mc[t];
+                if (ok[t]) mc[t] = *(const uint2*)(hmask + vox0 + xp * e2 + 256 * t);
+            }
+        if (xp < xb) w.load(xp + 1);
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                {
-                    float v = a[i];
-                    if (MODE == CONV_FWD_RELU) v = fmaxf(v + bias[4 * g + i], 0.f);
-                    if (MODE == CONV_BWD_MASK && hmask[vox * 16 + 4 * g + i] == 0) v = 0.f;
-                    o[i] = (short)f2bf(v);
-                }
-                *(s4*)(out + vox * 16 + 4 * g) = o;
+        for (int t = 0; t < 2; t++)
+        {
+            c2[t] = c1[t];
+            c1[t] = c0[t];
+            c0[t] = zero;
+            if (t && !two) continue;
+#pragma unroll
+            for (int k = 0; k < 5; k++)
+            {
+                const int at = k < 3 ? p0 + k * kLW * 8 : k == 3 ? q0 : q1;
+                const s8 bq  = *(const s8*)(buf + at + 16 * t * 8);
+                c2[t]        = mfma32(wa[2][k], bq, c2[t]);
+                c1[t]        = mfma32(wa[1][k], bq, c1[t]);
+                c0[t]        = mfma32(wa[0][k], bq, c0[t]);
             }
         }
-        __syncthreads();
+        if (xp > x0) emit(xp - 1, c2, mp);
     }
+    if (x1 == e) emit(e - 1, c1, mc);
 }
 
-// The first layer (1 -> 16 channels) with the scalar input staged in LDS
-// as for k_conv16_lds: a ring of 3 planes of (6 x 34) values; one 16x16x32
-// MFMA per 16-voxel tile covers all 27 taps (K = tap, lane group g holds taps
-// 8g..8g+7, the last 5 zero).  Bias and ReLU; BF16 out.
-template <typename TIN>
-__global__ void __launch_bounds__(256) k_conv1_lds(const TIN* __restrict__ in, const double* __restrict__ rms,
-    const uint16_t* __restrict__ wt, const float* __restrict__ bias, uint16_t* __restrict__ out, int e, int nyb,
-    int nzb)
+// A layer from one scalar per voxel to 16 channels: layer 0 (bias, ReLU), and
+// the backward pass of the last layer (times h > 0).  The scalars' planes are
+// BF16 in a ring of four (one barrier per plane); one 16x16x32 MFMA per
+// 16-voxel tile covers all 27 taps (lane group g holds taps 8g..8g+7, the
+// last five zero).  Inputs times 1 / rms (the box's normalised residual) when
+// rms is given.  Bound by the 32 bytes written per voxel: 256 boxes of 32^3
+// from FP64 (335 MB): 77 us (4.4 TB/s), 121 us with FP64 divisions, FP32
+// planes and two barriers per plane.
+template <typename TIN, int MODE>
+__global__ void __launch_bounds__(256) k_conv1(const TIN* __restrict__ in, const double* __restrict__ rms,
+    const uint16_t* __restrict__ wt, const float* __restrict__ bias, uint16_t* __restrict__ out,
+    const uint16_t* __restrict__ hmask, int e, int nyb, int nzb, int nxc, int xl)
 {
     constexpr int kP1 = kLH * kLW;
-    __shared__ float lds[3 * kP1];
-    const int b = blockIdx.x;
-    const int s = b / (nyb * nzb), yb = (b / nzb) % nyb, zb = b % nzb;
-    const int y0 = yb * kLY, z0 = zb * kLZ;
+    __shared__ uint16_t lds[4 * kP1];
+    int b        = blockIdx.x;
+    const int xc = b % nxc;
+    b /= nxc;
+    const int s = b / (nyb * nzb), y0 = (b / nzb) % nyb * kLY, z0 = b % nzb * kLZ;
+    const int x0 = xc * xl, x1 = min(e, x0 + xl);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
-    const int64_t e3 = (int64_t)e * e * e;
+    const int64_t e2 = (int64_t)e * e, e3 = e2 * e;
     const TIN* X = in + (int64_t)s * e3;
-    // inputs R / rms (the box's normalised residual) when rms is given
-    const double rs = rms ? rms[s] : 1.;
-    // A: W0[cout = n][taps 8g..8g+7] from the [16][32] layout
+    const double inv = rms ? 1. / rms[s] : 1.;
+    // A: W[cout = n][taps 8g..8g+7] from the [16][32] layout
     const s8 wa = *(const s8*)(wt + (size_t)n * 32 + 8 * g);
-    float bv4[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        bv4[i] = bias[4 * g + i];
-    auto stage = [&](int xp, int slot) {
-        float* dst = lds + slot * kP1;
-        for (int q = threadIdx.x; q < kP1; q += blockDim.x)
-        {
-            const int yy = q / kLW, zz = q - (q / kLW) * kLW;
-            const int y = y0 - 1 + yy, z = z0 - 1 + zz;
-            float v = 0.f;
-            if (xp >= 0 && xp < e && y >= 0 && y < e && z >= 0 && z < e)
-            {
-                const TIN r = X[((int64_t)xp * e + y) * e + z];
-                v           = rms ? (float)((double)r / rs) : (float)r;
-            }
-            dst[q] = v;
-        }
+    f4 bv = { 0.f, 0.f, 0.f, 0.f };
+    if (MODE == CONV_FWD_RELU) bv = *(const f4*)(bias + 4 * g);
+    // this thread's value of a plane's window
+    const int q = threadIdx.x, yy = q / kLW, ys = y0 - 1 + yy, zs = z0 - 1 + q - yy * kLW;
+    const bool in_w = q < kP1, in_box = in_w && ys >= 0 && ys < e && zs >= 0 && zs < e;
+    const int64_t at = (int64_t)ys * e + zs;
+    TIN r = 0;
+    auto load = [&](int xp) { r = in_box && xp >= 0 && xp < e ? X[xp * e2 + at] : (TIN)0; };
+    auto store = [&](int xp) {
+        if (in_w) lds[(xp & 3) * kP1 + q] = (uint16_t)cvt2(rms ? (float)((double)r * inv) : (float)r, 0.f);
     };
-    stage(-1, 2);
-    stage(0, 0);
-    const int y = y0 + wid;
-    for (int x = 0; x < e; x++)
+    // taps 8g..8g+7: plane and place in the window; the padding taps read the centre
+    int td[8], to[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++)
     {
-        stage(x + 1, (x + 1) % 3);
+        const int tap = 8 * g + i < kTaps ? 8 * g + i : 13;
+        td[i]         = tap_dx(tap);
+        to[i]         = (wid + 1 + tap_dy(tap)) * kLW + n + 1 + tap_dz(tap);
+    }
+    load(x0 - 1);
+    store(x0 - 1);
+    load(x0);
+    store(x0);
+    load(x0 + 1);
+    // this lane's outputs: voxels z0 + n (+ 16) of its row, channels 4g..4g+3
+    const int y        = y0 + wid;
+    const int64_t vox0 = ((int64_t)s * e3 + (int64_t)y * e + z0 + n) * 16 + 4 * g;
+    const bool ok[2]   = { y < e && z0 + n < e, y < e && z0 + 16 + n < e };
+    for (int x = x0; x < x1; x++)
+    {
+        store(x + 1);
+        const int64_t vox = vox0 + (int64_t)x * e2 * 16;
+        uint2 mask[2];
+        if (MODE == CONV_BWD_MASK)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+                if (ok[t]) mask[t] = *(const uint2*)(hmask + vox + 256 * t);
         __syncthreads();
-        s8 b0, b1;
+        if (x + 1 < x1) load(x + 2);
+        uint32_t u0[8], u1[8];
 #pragma unroll
         for (int i = 0; i < 8; i++)
         {
-            const int tap = 8 * g + i;
-            float v0 = 0.f, v1 = 0.f;
-            if (tap < kTaps)
-            {
-                const float* row = lds + ((x + 3 + tap_dx(tap)) % 3) * kP1 + (wid + 1 + tap_dy(tap)) * kLW;
-                const int zz     = n + 1 + tap_dz(tap);
-                v0               = row[zz];
-                v1               = row[zz + 16];
-            }
-            b0[i] = (short)f2bf(v0);
-            b1[i] = (short)f2bf(v1);
+            const uint16_t* p = lds + ((x + td[i]) & 3) * kP1 + to[i];
+            u0[i]             = p[0];
+            u1[i]             = p[16];
         }
+        uint4 v0, v1;
+        v0.x = u0[0] | u0[1] << 16, v0.y = u0[2] | u0[3] << 16, v0.z = u0[4] | u0[5] << 16, v0.w = u0[6] | u0[7] << 16;
+        v1.x = u1[0] | u1[1] << 16, v1.y = u1[2] | u1[3] << 16, v1.z = u1[4] | u1[5] << 16, v1.w = u1[6] | u1[7] << 16;
         const f4 z4 = { 0.f, 0.f, 0.f, 0.f };
-        const f4 acc0 = mfma32(wa, b0, z4), acc1 = mfma32(wa, b1, z4);
-        if (y < e)
+        const f4 acc[2] = { mfma32(wa, __builtin_bit_cast(s8, v0), z4), mfma32(wa, __builtin_bit_cast(s8, v1), z4) };
+#pragma unroll
+        for (int t = 0; t < 2; t++)
         {
+            if (!ok[t]) continue;
+            float v[4];
+            if (MODE == CONV_BWD_MASK)
+            {
+                const uint2 m = mask[t];
+                v[0] = m.x & 0xFFFFu ? acc[t][0] : 0.f;
+                v[1] = m.x >> 16 ? acc[t][1] : 0.f;
+                v[2] = m.y & 0xFFFFu ? acc[t][2] : 0.f;
+                v[3] = m.y >> 16 ? acc[t][3] : 0.f;
+            }
+            else
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    v[i] = fmaxf(acc[t][i] + bv[i], 0.f);
+            *(uint2*)(out + vox + 256 * t) = (uint2){ cvt2(v[0], v[1]), cvt2(v[2], v[3]) };
+        }
+    }
+}
+
+// The last layer (16 -> 1 channel).  A block owns rows y0..y0+7, z0..z0+31 and
+// marches along x like k_conv16, two rows per wave.  The rows of the MFMA are
+// the nine (dy, dx) of the taps, row 4(dy+1) + dx+1 (the others zero), and dz
+// and the channels its K: two MFMAs and two operand reads per 16 voxels of
+// input.  Lane group dy+1 then holds, in element dx+1, its share of the output
+// plane xp - dx: elements move up by one per plane (the accumulator of the
+// next), element 2 is complete, and the three groups' values of the rows y-1,
+// y, y+1 are added across the wave.
+// With R non-null it also finishes the network on the box: y = s x + z with
+// x = (float)(R / rms), written as (T)(y * rms) to out; otherwise z to zout.
+// Bound by HBM (32 bytes read per voxel).  256 boxes of 32^3 (403 MB): 90 us
+// (4.5 TB/s); 264 us with 27 taps of vector dot products from LDS.
+constexpr int kOY = 8, kOH = kOY + 2;
+template <typename T>
+__global__ void __launch_bounds__(256, 4) k_conv_out(const uint16_t* __restrict__ h, const uint16_t* __restrict__ wt,
+    const float* __restrict__ prm, float* __restrict__ zout, const double* __restrict__ R,
+    const double* __restrict__ rms, T* __restrict__ out, int e, int nyb, int nzb, int nxc, int xl)
+{
+    typedef Window<kOH> W;
+    __shared__ __align__(16) uint16_t lds[2][W::kSize];
+    int b        = blockIdx.x;
+    const int xc = b % nxc;
+    b /= nxc;
+    const int s = b / (nyb * nzb), y0 = (b / nzb) % nyb * kOY, z0 = b % nzb * kLZ;
+    const int x0 = xc * xl, x1 = min(e, x0 + xl);
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+    const int tsel = g >> 1, cs = 8 * (g & 1);
+    const int64_t e3 = (int64_t)e * e * e;
+    // A: row n = 4(dy+1) + dx+1; K = (dz = -1, 0) x 16, then dz = 1 (and zeros)
+    s8 wa[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+    {
+        const int dy = n >> 2, dx = n & 3;
+        const bool on = dy < 3 && dx < 3 && !(k && tsel);
+        const int tap = on ? (dx * 3 + dy) * 3 + (k ? 2 : tsel) : 0;
+        wa[k]         = *(const s8*)(wt + (size_t)tap * 256 + cs);
+        if (!on) wa[k] = (s8){ 0, 0, 0, 0, 0, 0, 0, 0 };
+    }
+    // the wave's rows: outputs y0+2wid, +1; inputs window rows 2wid .. 2wid+3
+    const int hb = (g & 1) * W::kHalf;
+    const int p0 = hb + (2 * wid * kLW + n + tsel) * 8, q0 = hb + (2 * wid * kLW + n + 2) * 8;
+    W w(h + (int64_t)s * e3 * 16, e, y0, z0);
+    const float bias = prm[kB3], sk = prm[kS];
+    const double rs = rms ? rms[s] : 1., inv = 1. / rs;
+    const bool two = z0 + 16 < e;
+    // lane (n, g) writes row g >> 1, z-tile g & 1 of the wave's four tiles
+    const int yo = y0 + 2 * wid + (g >> 1), zo = z0 + 16 * (g & 1) + n;
+    const bool store_ok = yo < e && zo < e;
+    const int64_t vox0 = (int64_t)s * e3 + (int64_t)yo * e + zo, e2 = (int64_t)e * e;
+    // writes plane x from element EL of the row tiles; rv: R there
+    auto emit = [&](auto EL, int x, const f4 (&c)[4][2], double rv) {
+        constexpr int el = decltype(EL)::value;
+        float mine       = 0.f;
+#pragma unroll
+        for (int r = 0; r < 2; r++)
 #pragma unroll
             for (int t = 0; t < 2; t++)
             {
-                const int z = z0 + 16 * t + n;
-                if (z >= e) continue;
-                const int64_t vox = (int64_t)s * e3 + ((int64_t)x * e + y) * e + z;
-                const f4 a = t == 0 ? acc0 : acc1;
-                s4 o;
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    o[i] = (short)f2bf(fmaxf(a[i] + bv4[i], 0.f));
-                *(s4*)(out + vox * 16 + 4 * g) = o;
+                const float a0 = c[r][t][el], a1 = c[r + 1][t][el], a2 = c[r + 2][t][el];
+                float v = g == 0 ? a0 : a1;
+                v       = g == 2 ? a2 : v;
+                v       = g == 3 ? 0.f : v;
+                v += __shfl_xor(v, 16, 64);
+                v += __shfl_xor(v, 32, 64);
+                mine = g == 2 * r + t ? v : mine;
             }
-        }
-        __syncthreads();
-    }
-}
-
-// The last layer (16 -> 1 channel) with the input staged in LDS: a block
-// owns rows y0..y0+7, z0..z0+31 of one sample (one voxel per thread) and
-// marches along x with a ring of 3 planes of (10 x 34) voxels; the 27 x 16
-// weights are LDS broadcasts of BF16 channel pairs, applied with the BF16
-// dot2 instruction (FP32 accumulation):
-//   z = b + sum_tap sum_ci W[tap][ci] h[v + off(tap)][ci]   (tap-major)
-// With R non-null it also finishes the network on the box: y = s x + z with
-// x = (float)(R / rms), written as (T)(y * rms) to out; otherwise z to zout.
-constexpr int kOY = 8, kOH = kOY + 2;
-template <typename T>
-__global__ void __launch_bounds__(256) k_conv_out_lds(const uint16_t* __restrict__ h, const uint16_t* __restrict__ wt,
-    const float* __restrict__ prm, float* __restrict__ zout, const double* __restrict__ R,
-    const double* __restrict__ rms, T* __restrict__ out, int e, int nyb, int nzb)
-{
-    constexpr int kPO = kOH * kLW * 16;
-    __shared__ __align__(16) uint16_t lds[3 * kPO];
-    __shared__ uint32_t w[kTaps * 8];  // channel pairs (2k, 2k+1) of W[tap], BF16
-    for (int q = threadIdx.x; q < kTaps * 8; q += blockDim.x)
-    {
-        const int tap = q / 8, k = q % 8;  // row 0 of the padded [27][16][16] layout
-        w[q] = (uint32_t)wt[tap * 256 + 2 * k] | ((uint32_t)wt[tap * 256 + 2 * k + 1] << 16);
-    }
-    const int b = blockIdx.x;
-    const int s = b / (nyb * nzb), yb = (b / nzb) % nyb, zb = b % nzb;
-    const int y0 = yb * kOY, z0 = zb * kLZ;
-    const int64_t e3 = (int64_t)e * e * e;
-    const uint16_t* X = h + (int64_t)s * e3 * 16;
-    auto stage = [&](int xp, int slot) {
-        uint4* dst = (uint4*)(lds + slot * kPO);
-        for (int q = threadIdx.x; q < kOH * kLW * 2; q += blockDim.x)
-        {
-            const int vox = q >> 1, half = q & 1;
-            const int yy = vox / kLW, zz = vox - (vox / kLW) * kLW;
-            const int y = y0 - 1 + yy, z = z0 - 1 + zz;
-            uint4 v = { 0u, 0u, 0u, 0u };
-            if (xp >= 0 && xp < e && y >= 0 && y < e && z >= 0 && z < e)
-                v = *(const uint4*)(X + (((int64_t)xp * e + y) * e + z) * 16 + 8 * half);
-            dst[q] = v;
-        }
+        if (!store_ok) return;
+        const float z = bias + mine;
+        if (R)
+            out[vox0 + x * e2] = (T)((double)(sk * (float)(rv * inv) + z) * rs);
+        else
+            zout[vox0 + x * e2] = z;
     };
-    stage(-1, 2);
-    stage(0, 0);
-    const int ry = threadIdx.x >> 5, rz = threadIdx.x & 31;
-    const int y = y0 + ry, z = z0 + rz;
-    const float bias = prm[kB3], sk = prm[kS];
-    const double rs  = rms ? rms[s] : 1.;
-    for (int x = 0; x < e; x++)
-    {
-        stage(x + 1, (x + 1) % 3);
-        __syncthreads();
-        float acc = bias;
-        for (int tap = 0; tap < kTaps; tap++)
-        {
-            const uint16_t* src = lds + ((x + 3 + tap_dx(tap)) % 3) * kPO
-                                  + ((ry + 1 + tap_dy(tap)) * kLW + (rz + 1 + tap_dz(tap))) * 16;
-            const uint4 a = ((const uint4*)src)[0], bq = ((const uint4*)src)[1];
-            const uint32_t u[8] = { a.x, a.y, a.z, a.w, bq.x, bq.y, bq.z, bq.w };
-            const uint32_t* wr  = w + tap * 8;
+    const f4 zero = { 0.f, 0.f, 0.f, 0.f };
+    f4 c[4][2];
 #pragma unroll
-            for (int k = 0; k < 8; k++)
-                acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, u[k]), __builtin_bit_cast(bf2, wr[k]),
-                    acc, false);
-        }
-        if (y < e && z < e)
-        {
-            const int64_t vox = (int64_t)s * e3 + ((int64_t)x * e + y) * e + z;
-            if (R)
+    for (int r = 0; r < 4; r++)
+        c[r][0] = c[r][1] = zero;
+    const int xa = max(x0 - 1, 0), xb = min(x1, e - 1);
+    double rp = 0., rc = 0.;  // R on planes xp - 1, xp: loaded a plane ahead of its use
+    w.load(xa);
+    for (int xp = xa; xp <= xb; xp++)
+    {
+        uint16_t* buf = lds[xp & 1];
+        w.store(buf);
+        __syncthreads();
+        rp = rc;
+        if (R && store_ok) rc = R[vox0 + xp * e2];
+        if (xp < xb) w.load(xp + 1);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
             {
-                const float xv = (float)(R[vox] / rs);
-                const float yv = sk * xv + acc;
-                out[vox]       = (T)((double)yv * rs);
+                if (t && !two) continue;
+                const s8 b0 = *(const s8*)(buf + p0 + (r * kLW + 16 * t) * 8);
+                const s8 b1 = *(const s8*)(buf + q0 + (r * kLW + 16 * t) * 8);
+                const f4 o  = c[r][t];
+                f4 d        = { 0.f, o[0], o[1], 0.f };
+                d           = mfma32(wa[0], b0, d);
+                c[r][t]     = mfma32(wa[1], b1, d);
             }
-            else
-                zout[vox] = acc;
-        }
-        __syncthreads();
+        if (xp > x0) emit(std::integral_constant<int, 2>(), xp - 1, c, rp);
     }
-}
-
-// The last layer (16 -> 1 channel) on the vector units: one output voxel per
-// thread, the 27 x 16 weights and the bias in LDS (FP32 values of the BF16
-// weights), two 16-byte loads per tap.  z = b + sum_tap sum_ci W[tap][ci] h[v + off(tap)][ci]
-// in FP32, as the MFMA path accumulates it.
-__global__ void __launch_bounds__(256) k_conv_out(const uint16_t* __restrict__ h, const uint16_t* __restrict__ wt,
-    const float* __restrict__ bias, float* __restrict__ out, int e, int64_t nvox)
-{
-    __shared__ float w[kTaps * 16];
-    for (int q = threadIdx.x; q < kTaps * 16; q += blockDim.x)
-        w[q] = bf2f(wt[(q / 16) * 256 + (q % 16)]);  // row 0 of the padded [27][16][16] layout
-    __syncthreads();
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nvox) return;
-    const int64_t e3 = (int64_t)e * e * e;
-    const int64_t s  = v / e3;
-    int r            = (int)(v - s * e3);
-    const int x = r / (e * e), y = (r / e) % e, z = r % e;
-    float acc = bias[0];
-    for (int tap = 0; tap < kTaps; tap++)
-    {
-        const int xi = x + tap_dx(tap), yi = y + tap_dy(tap), zi = z + tap_dz(tap);
-        if (xi < 0 || xi >= e || yi < 0 || yi >= e || zi < 0 || zi >= e) continue;
-        const uint4* p = (const uint4*)(h + (s * e3 + ((int64_t)xi * e + yi) * e + zi) * 16);
-        const uint4 a = p[0], b = p[1];
-        const uint32_t u[8] = { a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w };
-        const float* wr = w + tap * 16;
-#pragma unroll
-        for (int k = 0; k < 8; k++)
-        {
-            acc += wr[2 * k] * bf2f((uint16_t)(u[k] & 0xFFFFu));
-            acc += wr[2 * k + 1] * bf2f((uint16_t)(u[k] >> 16));
-        }
-    }
-    out[v] = acc;
+    if (x1 == e) emit(std::integral_constant<int, 1>(), e - 1, c, rc);
 }
 
 // The two halves of a dword pair (a in the low half)
@@ -908,25 +889,39 @@ __global__ void k_adam(float* p, const float* g, float* m, float* v, int n, floa
     p[q] -= lr * (mq / c1) / (sqrtf(vq / c2) + eps);
 }
 
-// per box: rms_j = sqrt(mean R_j^2) (0 -> 1); x = R/rms (FP32); t = KR/rms
-__global__ void __launch_bounds__(256) k_box_rms(const double* R, int64_t m, double* rms)
+// per box: rms_j = sqrt(mean R_j^2) (0 -> 1); x = R/rms (FP32); t = KR/rms.
+// One block of 16 waves per box with four loads in flight per thread: 256
+// boxes of 32^3 17 us (4 waves, one load at a time: 55 us)
+__global__ void __launch_bounds__(1024) k_box_rms(const double* R, int64_t m, double* rms)
 {
-    __shared__ double red[4];
-    const int j = blockIdx.x;
-    double a    = 0.;
-    for (int64_t i = threadIdx.x; i < m; i += blockDim.x)
+    __shared__ double red[16];
+    const double* r = R + (int64_t)blockIdx.x * m;
+    double a[4]     = { 0., 0., 0., 0. };
+    int64_t i       = threadIdx.x;
+    for (; i + 3 * 1024 < m; i += 4 * 1024)
     {
-        const double v = R[(int64_t)j * m + i];
-        a += v * v;
+        double v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            v[k] = r[i + 1024 * k];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            a[k] += v[k] * v[k];
     }
+    for (; i < m; i += 1024)
+        a[0] += r[i] * r[i];
+    double t = (a[0] + a[1]) + (a[2] + a[3]);
     for (int o = 32; o > 0; o >>= 1)
-        a += __shfl_xor(a, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a;
+        t += __shfl_xor(t, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
     __syncthreads();
     if (threadIdx.x == 0)
     {
-        const double r = sqrt((red[0] + red[1] + red[2] + red[3]) / (double)m);
-        rms[j]         = r > 0. ? r : 1.;
+        t = 0.;
+        for (int k = 0; k < 16; k++)
+            t += red[k];
+        t                = sqrt(t / (double)m);
+        rms[blockIdx.x] = t > 0. ? t : 1.;
     }
 }
 
@@ -971,9 +966,12 @@ namespace
 
 constexpr int kLossBlocks = 1024;
 
-// planes per x-chunk of a scalar layer's weight gradient: the columns alone
-// when they give four blocks per CU, else chunks of at least four planes
-int dw1_xl(int e, int64_t cols)
+// planes per x-chunk of a marching kernel with `cols` columns of blocks: the
+// whole edge when they alone give four blocks per CU (what the registers of
+// k_conv16 let reside), else chunks of at least four planes (each reads a plane
+// more on either side).  64 boxes of 32^3, k_conv16: 37 us in two chunks, 47 us
+// in one
+int march_xl(int e, int64_t cols)
 {
     const int64_t want = std::max<int64_t>(1, std::min<int64_t>(1024 / cols, (e + 3) / 4));
     return (int)((e + want - 1) / want);
@@ -985,8 +983,6 @@ int64_t dw1_blocks(int e, int max_batch)
     const int64_t per = (int64_t)((e + kSY - 1) / kSY) * ((e + kLZ - 1) / kLZ);
     return std::max<int64_t>(1024 + per, per * max_batch);
 }
-
-int64_t ntiles(int e, int nb) { return (int64_t)nb * e * e * ((e + 15) / 16); }
 
 int derive(mgx_cnn* c)
 {
@@ -1009,21 +1005,23 @@ int forward_any(mgx_cnn* c, const float* x, const double* R, const double* rms, 
     int rc;
     if ((rc = derive(c))) return rc;
     const int e   = c->edge;
-    const int nyb = (e + kLY - 1) / kLY, nzb = (e + kLZ - 1) / kLZ;
-    const dim3 lgrid((unsigned)(nb * nyb * nzb));
+    const int nyb = (e + kLY - 1) / kLY, nzb = (e + kLZ - 1) / kLZ, cols = nb * nyb * nzb;
+    const int xl = march_xl(e, cols), nxc = (e + xl - 1) / xl;
+    const dim3 lgrid((unsigned)(cols * nxc));
+    const uint16_t* nomask = nullptr;
     if (R)
-        hipLaunchKernelGGL(k_conv1_lds<double>, lgrid, dim3(256), 0, ctx->stream, R, rms, (const uint16_t*)c->f0,
-            (const float*)c->p + kB0, c->h1, e, nyb, nzb);
+        hipLaunchKernelGGL((k_conv1<double, CONV_FWD_RELU>), lgrid, dim3(256), 0, ctx->stream, R, rms,
+            (const uint16_t*)c->f0, (const float*)c->p + kB0, c->h1, nomask, e, nyb, nzb, nxc, xl);
     else
-        hipLaunchKernelGGL(k_conv1_lds<float>, lgrid, dim3(256), 0, ctx->stream, x, (const double*)nullptr,
-            (const uint16_t*)c->f0, (const float*)c->p + kB0, c->h1, e, nyb, nzb);
-    hipLaunchKernelGGL((k_conv16_lds<CONV_FWD_RELU>), lgrid, dim3(256), 0, ctx->stream, (const uint16_t*)c->h1,
-        (const uint16_t*)c->f1, (const float*)c->p + kB1, c->h2, (const uint16_t*)nullptr, e, nyb, nzb);
-    hipLaunchKernelGGL((k_conv16_lds<CONV_FWD_RELU>), lgrid, dim3(256), 0, ctx->stream, (const uint16_t*)c->h2,
-        (const uint16_t*)c->f2, (const float*)c->p + kB2, c->h3, (const uint16_t*)nullptr, e, nyb, nzb);
-    const int noy = (e + kOY - 1) / kOY;
-    hipLaunchKernelGGL(k_conv_out_lds<T>, dim3((unsigned)(nb * noy * nzb)), dim3(256), 0, ctx->stream,
-        (const uint16_t*)c->h3, (const uint16_t*)c->f3, (const float*)c->p, c->z, R, rms, out, e, noy, nzb);
+        hipLaunchKernelGGL((k_conv1<float, CONV_FWD_RELU>), lgrid, dim3(256), 0, ctx->stream, x, (const double*)nullptr,
+            (const uint16_t*)c->f0, (const float*)c->p + kB0, c->h1, nomask, e, nyb, nzb, nxc, xl);
+    hipLaunchKernelGGL((k_conv16<CONV_FWD_RELU>), lgrid, dim3(256), 0, ctx->stream, (const uint16_t*)c->h1,
+        (const uint16_t*)c->f1, (const float*)c->p + kB1, c->h2, nomask, e, nyb, nzb, nxc, xl);
+    hipLaunchKernelGGL((k_conv16<CONV_FWD_RELU>), lgrid, dim3(256), 0, ctx->stream, (const uint16_t*)c->h2,
+        (const uint16_t*)c->f2, (const float*)c->p + kB2, c->h3, nomask, e, nyb, nzb, nxc, xl);
+    const int noy = (e + kOY - 1) / kOY, ocols = nb * noy * nzb, oxl = march_xl(e, ocols), onx = (e + oxl - 1) / oxl;
+    hipLaunchKernelGGL(k_conv_out<T>, dim3((unsigned)(ocols * onx)), dim3(256), 0, ctx->stream,
+        (const uint16_t*)c->h3, (const uint16_t*)c->f3, (const float*)c->p, c->z, R, rms, out, e, noy, nzb, onx, oxl);
     MGX_CHECK_LAUNCH(ctx);
     return MGX_OK;
 }
@@ -1057,7 +1055,7 @@ int dw1(mgx_cnn* c, const uint16_t* ch, const float* sc, int nb, float* part, Dw
 {
     mgx_ctx* ctx  = c->ctx;
     const int e   = c->edge, nyb = (e + kSY - 1) / kSY, nzb = (e + kLZ - 1) / kLZ, cols = nb * nyb * nzb;
-    const int xl  = dw1_xl(e, cols), nxc = (e + xl - 1) / xl;
+    const int xl  = march_xl(e, cols), nxc = (e + xl - 1) / xl;
     hipLaunchKernelGGL(k_dw1<FLIP>, dim3(cols * nxc), dim3(256), 0, ctx->stream, ch, sc, e, nyb, nzb, nxc, xl, part);
     MGX_CHECK_LAUNCH(ctx);
     l.part = part, l.np = cols * nxc, l.nw = kTaps * 16, l.nb = FLIP ? 0 : 16, l.stride = kTaps * 16 + 16;
@@ -1070,9 +1068,8 @@ int grad(mgx_cnn* c, const float* x, const float* t, int nb, double* loss)
     mgx_ctx* ctx = c->ctx;
     int rc;
     if ((rc = forward(c, x, nb))) return rc;
-    const int e = c->edge, nzt = (e + 15) / 16;
-    const int64_t n  = (int64_t)nb * e * e * e;
-    const int64_t nt = ntiles(e, nb);
+    const int e     = c->edge;
+    const int64_t n = (int64_t)nb * e * e * e;
     hipLaunchKernelGGL(k_loss, dim3(kLossBlocks), dim3(256), 0, ctx->stream, x, (const float*)c->z, t,
         (const float*)c->p, n, (float*)nullptr, c->dy, c->lpart);
     hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(192), 0, ctx->stream, (const double*)c->lpart, kLossBlocks, c->g,
@@ -1082,23 +1079,24 @@ int grad(mgx_cnn* c, const float* x, const float* t, int nb, double* loss)
     // layer 3: dZ3 = dy (scalar; its bias came with the loss)
     if ((rc = dw1<true>(c, c->h3, c->dy, nb, c->part3, L.l[3]))) return rc;
     L.l[3].gw = c->g + kW3, L.l[3].gb = nullptr;
-    const dim3 grid((unsigned)((nt + kWaves - 1) / kWaves)), blk(64 * kWaves);
-    hipLaunchKernelGGL((k_conv<1, 16, CONV_BWD_MASK>), grid, blk, 0, ctx->stream, (const void*)c->dy, c->r3,
-        (const float*)nullptr, (void*)c->dza, (const uint16_t*)c->h3, e, nzt, nt);
+    const int nyb = (e + kLY - 1) / kLY, nzb = (e + kLZ - 1) / kLZ, cols = nb * nyb * nzb;
+    const int xl = march_xl(e, cols), nxc = (e + xl - 1) / xl;
+    const dim3 lgrid((unsigned)(cols * nxc));
+    const float* nobias = nullptr;
+    hipLaunchKernelGGL((k_conv1<float, CONV_BWD_MASK>), lgrid, dim3(256), 0, ctx->stream, (const float*)c->dy,
+        (const double*)nullptr, (const uint16_t*)c->r3, nobias, c->dza, (const uint16_t*)c->h3, e, nyb, nzb, nxc, xl);
     MGX_CHECK_LAUNCH(ctx);
     // layer 2: dZ2 = dza
     if ((rc = dw16(c, c->dza, c->h2, nb, c->part2, L.l[2]))) return rc;
     L.l[2].gw = c->g + kW2, L.l[2].gb = c->g + kB2;
-    const int nyb = (e + kLY - 1) / kLY, nzb = (e + kLZ - 1) / kLZ;
-    const dim3 lgrid((unsigned)(nb * nyb * nzb));
-    hipLaunchKernelGGL((k_conv16_lds<CONV_BWD_MASK>), lgrid, dim3(256), 0, ctx->stream, (const uint16_t*)c->dza,
-        (const uint16_t*)c->r2, (const float*)nullptr, c->dzb, (const uint16_t*)c->h2, e, nyb, nzb);
+    hipLaunchKernelGGL((k_conv16<CONV_BWD_MASK>), lgrid, dim3(256), 0, ctx->stream, (const uint16_t*)c->dza,
+        (const uint16_t*)c->r2, nobias, c->dzb, (const uint16_t*)c->h2, e, nyb, nzb, nxc, xl);
     MGX_CHECK_LAUNCH(ctx);
     // layer 1: dZ1 = dzb
     if ((rc = dw16(c, c->dzb, c->h1, nb, c->part1, L.l[1]))) return rc;
     L.l[1].gw = c->g + kW1, L.l[1].gb = c->g + kB1;
-    hipLaunchKernelGGL((k_conv16_lds<CONV_BWD_MASK>), lgrid, dim3(256), 0, ctx->stream, (const uint16_t*)c->dzb,
-        (const uint16_t*)c->r1, (const float*)nullptr, c->dza, (const uint16_t*)c->h1, e, nyb, nzb);
+    hipLaunchKernelGGL((k_conv16<CONV_BWD_MASK>), lgrid, dim3(256), 0, ctx->stream, (const uint16_t*)c->dzb,
+        (const uint16_t*)c->r1, nobias, c->dza, (const uint16_t*)c->h1, e, nyb, nzb, nxc, xl);
     MGX_CHECK_LAUNCH(ctx);
     // layer 0: dZ0 = dza, input x
     if ((rc = dw1<false>(c, c->dza, x, nb, c->part0, L.l[0]))) return rc;
@@ -1273,7 +1271,7 @@ int mgx_cnn_make_pairs(mgx_cnn* c, int nbox, const double* R, const double* KR, 
     const int64_t m = (int64_t)c->edge * c->edge * c->edge;
     double* rms     = nullptr;
     MGX_CHECK_HIP(ctx, hipMalloc((void**)&rms, (size_t)nbox * sizeof(double)));
-    hipLaunchKernelGGL(k_box_rms, dim3(nbox), dim3(256), 0, ctx->stream, R, m, rms);
+    hipLaunchKernelGGL(k_box_rms, dim3(nbox), dim3(1024), 0, ctx->stream, R, m, rms);
     hipLaunchKernelGGL(k_box_scale_to_f32, dim3(4096), dim3(256), 0, ctx->stream, R, (const double*)rms, m,
         m * nbox, x);
     hipLaunchKernelGGL(k_box_scale_to_f32, dim3(4096), dim3(256), 0, ctx->stream, KR, (const double*)rms, m,
@@ -1300,7 +1298,7 @@ int cnn_apply_boxes(mgx_cnn* c, int nbox, int edge, const double* R, void* out, 
     {
         const int nb     = std::min(c->max_batch, nbox - b0);
         const double* Rb = R + (int64_t)b0 * m;
-        hipLaunchKernelGGL(k_box_rms, dim3(nb), dim3(256), 0, ctx->stream, Rb, m, c->rms);
+        hipLaunchKernelGGL(k_box_rms, dim3(nb), dim3(1024), 0, ctx->stream, Rb, m, c->rms);
         MGX_CHECK_LAUNCH(ctx);
         rc = out_dtype == MGX_F32
                  ? forward_any<float>(c, nullptr, Rb, c->rms, nb, (float*)out + (int64_t)b0 * m)

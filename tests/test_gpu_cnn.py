@@ -49,6 +49,33 @@ def test_cnn_forward_matches_oracle(ctx, edge, nb):
     net.close()
 
 
+@pytest.mark.parametrize("edge,nb", [(1, 2), (3, 2), (8, 1), (9, 2), (17, 1), (33, 1), (40, 1), (12, 9)])
+def test_cnn_forward_and_apply_edges(ctx, edge, nb):
+    """Edges around the kernels' tiles (16 and 32 z-voxels, 4 and 8 rows, chunks
+    of 4 and more planes), one sample and several, through the training forward
+    and the box apply (batches of at most two boxes, the last one ragged).
+    BF16 rounding points as in the oracle: 5e-3 as in the test above."""
+    p = _params(4)
+    rng = np.random.default_rng(1000 + edge)
+    x = rng.standard_normal((nb, edge, edge, edge)).astype(np.float32)
+    net = learned.Cnn(ctx, edge, nb, p)
+    ty = to_dev(np.zeros_like(x))
+    net.forward(to_dev(x), nb, ty)
+    ref, _ = OC.forward(p, x, bf16_mode=True)
+    assert _rel(to_np(ty), ref) < 5e-3
+    net.close()
+    R = x.astype(np.float64) * 10.0 ** -np.arange(nb)[:, None, None, None]
+    rms = np.sqrt(np.mean(R * R, axis=(1, 2, 3)))[:, None, None, None]
+    net = learned.Cnn(ctx, edge, min(nb, 2), p)
+    to = to_dev(np.zeros_like(R))
+    net.apply(nb, to_dev(R), to)
+    ref, _ = OC.forward(p, (R / rms).astype(np.float32), bf16_mode=True)
+    out = to_np(to) / rms
+    for j in range(nb):
+        assert _rel(out[j], ref[j]) < 5e-3, j
+    net.close()
+
+
 def test_cnn_grad_matches_oracle(ctx):
     p = _params(2)
     rng = np.random.default_rng(7)

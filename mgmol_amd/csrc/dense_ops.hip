@@ -2,17 +2,18 @@
 //
 // ss(i,j) = vel * sum_k A(k,i) B(k,j) over one slab of rows (the reference's
 // per-subdomain LocalMatrices, src/LocGridOrbitals.cc:1504-1604).  Each wave
-// owns one 16x16 output tile and a chunk of rows:
+// owns the tiles of one pair of column panels and every so many 16-row chunks:
 //   PREC_F64  : v_mfma_f64_16x16x4_f64, FP64 accumulation;
 //   PREC_SPLIT: x = hi + lo (hi = fl32(x), lo = fl32(x - hi)),
 //               v_mfma_f32_16x16x4_f32 on hi*hi and hi*lo + lo*hi, FP32
-//               accumulation over 64-row sub-chunks, FP64 sum of sub-chunks.
+//               accumulation over 16 rows, FP64 sums of those.
 // Chunk partials are reduced in a fixed order (deterministic) and scaled.
 #include "common.hpp"
 
 #include <rocsolver/rocsolver.h>
 
 #include <mutex>
+#include <type_traits>
 
 namespace mgx
 {
@@ -28,107 +29,242 @@ constexpr int kWaves = 4;  // waves per block, each on its own row sub-chunk
 // and B[k=l/16][n=l%16].  Accumulator v of lane l holds D[4*(l/16)+v][l%16]
 // for v_mfma_f32_16x16x4_f32 and D[l/16+4*v][l%16] for v_mfma_f64_16x16x4_f64
 // (both checked on gfx950 by tests/test_gpu_dense.py).
-template <int PREC>
-__global__ void __launch_bounds__(64 * kWaves) k_tsgemm(const double* A, const double* B, int64_t ld,
-    int64_t loc_numpt, int n, int ntile, int nchunk, int64_t rows_per_chunk, int lower_only, double* part)
+// Panels of TW 16-column tiles: a wave holds the TW x TW output tiles of one
+// panel pair for its share of the rows (all of an output up to 64 columns, so
+// each operand is read once) and reads its columns straight from memory: lane
+// (c, r) takes rows 4r..4r+3 of a 16-row chunk of column c (32 bytes; a column's
+// 16 rows are 128 contiguous bytes), which the MFMAs take as their four steps
+// (a product does not care which row is which k, as long as A and B agree).
+// The next chunk's loads are in flight during the MFMAs.  The four waves of a
+// block take neighbouring chunks and add their tiles through LDS in order.
+//   PREC_F64  : TW^2 (a Gram's diagonal pair: the lower tiles) MFMAs per step;
+//   PREC_SPLIT: hi * hi and hi * lo + lo * hi in FP32 over the 16 rows, added
+//               in FP64.
+// Bound by the FP64 matrix rate and HBM together.  64 columns of 884736 rows:
+// Gram 107 us (4.2 TB/s), product 170 us (5.3 TB/s, 43 TFLOP/s); 16x16 tiles of
+// scattered 8-byte loads took 852 us each.
+template <int PREC, int TW, bool DIAG, bool VEC>
+__device__ __forceinline__ void tsgemm_panels(const double* A, const double* B, int64_t ld, int64_t k_begin,
+    int64_t lnp, int n, int i0, int j0, int chunk, int nchunk, double* red, double* out)
 {
-    const int tile  = blockIdx.x;  // tile index over (ti, tj)
-    const int chunk = blockIdx.y;
-    const int slab  = blockIdx.z;
-    const int ti = tile / ntile, tj = tile - (tile / ntile) * ntile;
-    if (lower_only && tj > ti) return;
-    const int lane = threadIdx.x & 63;
-    const int wid  = threadIdx.x >> 6;
-    const int c = lane & 15, r = lane >> 4;
-    const int i0 = ti * 16, j0 = tj * 16;
-    const int64_t k_begin = (int64_t)slab * loc_numpt + (int64_t)chunk * rows_per_chunk;
-    int64_t k_end         = k_begin + rows_per_chunk;
-    const int64_t slab_end = (int64_t)(slab + 1) * loc_numpt;
-    if (k_end > slab_end) k_end = slab_end;
-    const int ia = i0 + c, jb = j0 + c;
-    const bool va = ia < n, vb = jb < n;
-    const double* pa = A + (int64_t)(va ? ia : 0) * ld;
-    const double* pb = B + (int64_t)(vb ? jb : 0) * ld;
-    // the wave's rows: interleave waves in blocks of 64 rows
-    double acc[4] = { 0., 0., 0., 0. };
-    if (PREC == MGX_PREC_F64)
+    typedef double dd2 __attribute__((ext_vector_type(2)));
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, c = lane & 15, r = lane >> 4;
+    const double *pa[TW], *pb[TW];
+#pragma unroll
+    for (int q = 0; q < TW; q++)
     {
-        d4 d = { 0., 0., 0., 0. };
-        for (int64_t k0 = k_begin + 64 * wid; k0 < k_end; k0 += 64 * kWaves)
-        {
-#pragma unroll 4
-            for (int s = 0; s < 16; s++)
-            {
-                const int64_t k = k0 + 4 * s + r;
-                const bool in   = k < k_end;
-                const double a  = (va && in) ? pa[k] : 0.;
-                const double b  = (vb && in) ? pb[k] : 0.;
-                d = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, d, 0, 0, 0);
-            }
-        }
-        for (int v = 0; v < 4; v++)
-            acc[v] = d[v];
+        // columns past n repeat the last one; their results are not written
+        pa[q] = A + (int64_t)min(i0 + 16 * q + c, n - 1) * ld + k_begin + 4 * r;
+        pb[q] = B + (int64_t)min(j0 + 16 * q + c, n - 1) * ld + k_begin + 4 * r;
     }
-    else
+    struct Frag
     {
-        for (int64_t k0 = k_begin + 64 * wid; k0 < k_end; k0 += 64 * kWaves)
+        double v[TW][4];
+    };
+    auto load = [&](Frag& f, const double* const (&p)[TW], int64_t k) {
+#pragma unroll
+        for (int q = 0; q < TW; q++)
         {
-            f4 hh = { 0.f, 0.f, 0.f, 0.f }, hx = { 0.f, 0.f, 0.f, 0.f };
-#pragma unroll 4
-            for (int s = 0; s < 16; s++)
+            if (VEC)
             {
-                const int64_t k = k0 + 4 * s + r;
-                const bool in   = k < k_end;
-                const double a  = (va && in) ? pa[k] : 0.;
-                const double b  = (vb && in) ? pb[k] : 0.;
-                const float ah = (float)a, al = (float)(a - (double)ah);
-                const float bh = (float)b, bl = (float)(b - (double)bh);
-                hh = __builtin_amdgcn_mfma_f32_16x16x4f32(ah, bh, hh, 0, 0, 0);
-                hx = __builtin_amdgcn_mfma_f32_16x16x4f32(ah, bl, hx, 0, 0, 0);
-                hx = __builtin_amdgcn_mfma_f32_16x16x4f32(al, bh, hx, 0, 0, 0);
+                const dd2 x = *(const dd2*)(p[q] + k), y = *(const dd2*)(p[q] + k + 2);
+                f.v[q][0] = x[0], f.v[q][1] = x[1], f.v[q][2] = y[0], f.v[q][3] = y[1];
             }
-            for (int v = 0; v < 4; v++)
-                acc[v] += (double)hh[v] + (double)hx[v];
+            else
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+                    f.v[q][s] = p[q][k + s];
+        }
+    };
+    d4 acc[TW][TW];
+#pragma unroll
+    for (int x = 0; x < TW; x++)
+#pragma unroll
+        for (int y = 0; y < TW; y++)
+            acc[x][y] = (d4){ 0., 0., 0., 0. };
+    auto mul = [&](const Frag& a, const Frag& b) {
+        if (PREC == MGX_PREC_F64)
+        {
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int x = 0; x < TW; x++)
+#pragma unroll
+                    for (int y = 0; y < TW; y++)
+                        if (!DIAG || y <= x)
+                            acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.v[x][s], b.v[y][s], acc[x][y], 0, 0, 0);
+            return;
+        }
+        float ah[TW][4], al[TW][4], bh[TW][4], bl[TW][4];
+#pragma unroll
+        for (int q = 0; q < TW; q++)
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+            {
+                ah[q][s] = (float)a.v[q][s];
+                al[q][s] = (float)(a.v[q][s] - (double)ah[q][s]);
+                bh[q][s] = DIAG ? ah[q][s] : (float)b.v[q][s];
+                bl[q][s] = DIAG ? al[q][s] : (float)(b.v[q][s] - (double)bh[q][s]);
+            }
+#pragma unroll
+        for (int x = 0; x < TW; x++)
+#pragma unroll
+            for (int y = 0; y < TW; y++)
+            {
+                if (DIAG && y > x) continue;
+                f4 hh = { 0.f, 0.f, 0.f, 0.f }, hx = { 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+                {
+                    hh = __builtin_amdgcn_mfma_f32_16x16x4f32(ah[x][s], bh[y][s], hh, 0, 0, 0);
+                    hx = __builtin_amdgcn_mfma_f32_16x16x4f32(ah[x][s], bl[y][s], hx, 0, 0, 0);
+                    hx = __builtin_amdgcn_mfma_f32_16x16x4f32(al[x][s], bh[y][s], hx, 0, 0, 0);
+                }
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    acc[x][y][v] += (double)hh[v] + (double)hx[v];
+            }
+    };
+    // full 16-row chunks first, first + step, ...
+    const int64_t nfull = lnp / 16, first = (int64_t)chunk * kWaves + wid, step = (int64_t)nchunk * kWaves;
+    Frag a0, b0, a1, b1;
+    if (first < nfull)
+    {
+        load(a0, pa, 16 * first);
+        if (!DIAG) load(b0, pb, 16 * first);
+        for (int64_t ch = first;;)
+        {
+            // the last chunk is loaded again where there is no next one
+            int64_t nx = ch + step, at = nx < nfull ? nx : ch;
+            load(a1, pa, 16 * at);
+            if (!DIAG) load(b1, pb, 16 * at);
+            mul(a0, DIAG ? a0 : b0);
+            if (nx >= nfull) break;
+            ch = nx;
+            nx = ch + step, at = nx < nfull ? nx : ch;
+            load(a0, pa, 16 * at);
+            if (!DIAG) load(b0, pb, 16 * at);
+            mul(a1, DIAG ? a1 : b1);
+            if (nx >= nfull) break;
+            ch = nx;
         }
     }
-    // combine the waves' partial tiles in LDS (fixed order)
-    __shared__ double red[kWaves][64][4];
-    for (int v = 0; v < 4; v++)
-        red[wid][lane][v] = acc[v];
-    __syncthreads();
-    if (wid == 0)
+    // the remaining lnp % 16 rows, by the wave whose turn it is
+    if (nfull * 16 < lnp && nfull % step == first)
     {
-        for (int v = 0; v < 4; v++)
+#pragma unroll
+        for (int q = 0; q < TW; q++)
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+            {
+                const bool in = nfull * 16 + 4 * r + s < lnp;
+                a0.v[q][s]    = in ? pa[q][nfull * 16 + s] : 0.;
+                if (!DIAG) b0.v[q][s] = in ? pb[q][nfull * 16 + s] : 0.;
+            }
+        mul(a0, DIAG ? a0 : b0);
+    }
+    // the waves' tiles, added in wave order
+    for (int w = 0; w < kWaves; w++)
+    {
+        if (wid == w)
         {
-            double s = red[0][lane][v];
-            for (int w = 1; w < kWaves; w++)
-                s += red[w][lane][v];
-            const int row = (PREC == MGX_PREC_F64) ? i0 + r + 4 * v : i0 + 4 * r + v;
-            const int col = j0 + c;
-            if (row < n && col < n)
-                part[(((int64_t)slab * nchunk + chunk) * n + col) * n + row] = s;
+#pragma unroll
+            for (int x = 0; x < TW; x++)
+#pragma unroll
+                for (int y = 0; y < TW; y++)
+                {
+                    if (DIAG && y > x) continue;
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                    {
+                        double* p      = red + ((x * TW + y) * 4 + v) * 64 + lane;
+                        const double t = w == 0 ? acc[x][y][v] : *p + acc[x][y][v];
+                        if (w < kWaves - 1)
+                            *p = t;
+                        else
+                        {
+                            const int row = i0 + 16 * x + (PREC == MGX_PREC_F64 ? r + 4 * v : 4 * r + v);
+                            const int col = j0 + 16 * y + c;
+                            if (row < n && col < n) out[(int64_t)col * n + row] = t;
+                        }
+                    }
+                }
         }
+        if (w < kWaves - 1) __syncthreads();
     }
 }
 
-// ss[slab](i,j) = vel * sum_chunks part; lower_only fills the upper triangle
-// from the lower one (SquareLocalMatrices::fillUpperWithLower)
-__global__ void k_chunk_reduce(const double* part, int n, int nchunk, int subdivx, double vel, int lower_only,
-    double* ss)
+template <int PREC, int TW, bool VEC>
+__global__ void __launch_bounds__(64 * kWaves, TW >= 3 ? 1 : 2) k_tsgemm(const double* A, const double* B, int64_t ld,
+    int64_t lnp, int n, int npan, int nchunk, int lower_only, double* part)
 {
-    const int64_t nn = (int64_t)n * n;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < nn * subdivx;
-         t += (int64_t)gridDim.x * blockDim.x)
+    __shared__ double red[TW * TW * 256];
+    const int chunk = blockIdx.x % nchunk, pair = blockIdx.x / nchunk, slab = blockIdx.z;
+    int ti, tj;
+    if (lower_only)
     {
-        const int64_t slab = t / nn;
-        const int64_t e    = t - slab * nn;
-        int col = (int)(e / n), row = (int)(e - (e / n) * n);
-        int64_t src = e;
-        if (lower_only && col > row) src = (int64_t)row * n + col;  // (col,row) element in col-major
+        // pairs on and below the diagonal, row by row
+        ti = 0;
+        while ((ti + 1) * (ti + 2) / 2 <= pair)
+            ti++;
+        tj = pair - ti * (ti + 1) / 2;
+    }
+    else
+    {
+        ti = pair / npan;
+        tj = pair - ti * npan;
+    }
+    const int64_t k0 = (int64_t)slab * lnp;
+    double* out      = part + ((int64_t)slab * nchunk + chunk) * n * n;
+    if (lower_only && ti == tj)
+        tsgemm_panels<PREC, TW, true, VEC>(A, A, ld, k0, lnp, n, ti * 16 * TW, tj * 16 * TW, chunk, nchunk, red, out);
+    else
+        tsgemm_panels<PREC, TW, false, VEC>(A, B, ld, k0, lnp, n, ti * 16 * TW, tj * 16 * TW, chunk, nchunk, red, out);
+}
+
+// ss[slab](i,j) = vel * sum_chunks part; lower_only fills the upper triangle
+// from the lower one (SquareLocalMatrices::fillUpperWithLower).  A block takes
+// 32 neighbouring entries, eight groups of threads every eighth partial each,
+// 16 loads in flight; the groups are added in order.  64 x 64 entries of 256
+// partials: 8 us; one thread per entry took 101 us (a chain of loads).
+__global__ void __launch_bounds__(256) k_chunk_reduce(const double* part, int n, int nchunk, int subdivx, double vel,
+    int lower_only, double* ss)
+{
+    __shared__ double red[8][32];
+    const int64_t nn = (int64_t)n * n, nt = (nn + 31) / 32;
+    const int col32 = threadIdx.x & 31, grp = threadIdx.x >> 5;
+    for (int64_t t = blockIdx.x; t < nt * subdivx; t += gridDim.x)
+    {
+        const int64_t slab = t / nt, e = (t - slab * nt) * 32 + col32;
         double s = 0.;
-        for (int c = 0; c < nchunk; c++)
-            s += part[(slab * nchunk + c) * nn + src];
-        ss[slab * nn + e] = s * vel;
+        if (e < nn)
+        {
+            const int col = (int)(e / n), row = (int)(e - (int64_t)col * n);
+            // (col,row) element in col-major above the diagonal
+            const double* p = part + slab * nchunk * nn + (lower_only && col > row ? (int64_t)row * n + col : e);
+            int c           = grp;
+            for (; c + 120 < nchunk; c += 128)
+            {
+                double v[16];
+#pragma unroll
+                for (int k = 0; k < 16; k++)
+                    v[k] = p[(c + 8 * k) * nn];
+#pragma unroll
+                for (int k = 0; k < 16; k++)
+                    s += v[k];
+            }
+            for (; c < nchunk; c += 8)
+                s += p[c * nn];
+        }
+        red[grp][col32] = s;
+        __syncthreads();
+        if (grp == 0 && e < nn)
+        {
+            for (int g = 1; g < 8; g++)
+                s += red[g][col32];
+            ss[slab * nn + e] = s * vel;
+        }
+        __syncthreads();
     }
 }
 
@@ -749,8 +885,8 @@ int tsgemm_wide(mgx_ctx* ctx, int prec, const double* A, const double* B, int64_
         hipLaunchKernelGGL(k_tsgemm_split_wide, grid, blk, 0, ctx->stream, As, Bs, ld, lnp, n, ntile, rps,
             same ? 1 : 0, parts);
         MGX_CHECK_LAUNCH(ctx);
-        hipLaunchKernelGGL(k_chunk_reduce, dim3(nblocks(nn)), dim3(kBlock), 0, ctx->stream, (const double*)parts, n,
-            nsplit, 1, vel, same ? 1 : 0, C);
+        hipLaunchKernelGGL(k_chunk_reduce, dim3(nblocks((nn + 31) / 32, 1)), dim3(256), 0, ctx->stream,
+            (const double*)parts, n, nsplit, 1, vel, same ? 1 : 0, C);
         MGX_CHECK_LAUNCH(ctx);
     }
     return MGX_OK;
@@ -765,12 +901,14 @@ int tsgemm(mgx_ctx* ctx, int prec, const double* A, const double* B, int64_t ld,
     MGX_REQUIRE(ctx, (int64_t)subdivx * lnp <= ld, "slabs exceed the leading dimension");
     MGX_REQUIRE(ctx, prec == MGX_PREC_F64 || prec == MGX_PREC_SPLIT, "bad precision mode");
     if (n >= kWideN) return tsgemm_wide(ctx, prec, A, B, ld, lnp, n, subdivx, vel, ss);
-    const int ntile  = (n + 15) / 16;
-    const int ntiles = ntile * ntile;
-    // enough chunks to fill the chip, each at least 256 rows
-    int64_t want = (4096 + ntiles - 1) / ntiles;
-    int64_t maxc = (lnp + 255) / 256;
-    int nchunk   = (int)std::max<int64_t>(1, std::min<int64_t>(want, maxc));
+    // the fewest panels of at most four tiles, all of one width
+    const int ntile = (n + 15) / 16, npan = (ntile + 3) / 4, tw = (ntile + npan - 1) / npan;
+    const int pairs = lower_only ? npan * (npan + 1) / 2 : npan * npan;
+    // blocks of four waves: as many per CU as the tiles' registers let reside
+    // (1, 2, 3, 6 for widths 4..1), each wave at least four chunks of 16 rows
+    static const int percu[4] = { 6, 3, 2, 1 };
+    const int64_t want = (256 * percu[tw - 1] + (int64_t)pairs * subdivx - 1) / ((int64_t)pairs * subdivx);
+    int nchunk         = (int)std::max<int64_t>(1, std::min<int64_t>(want, lnp / 256));
     const size_t per_chunk = (size_t)subdivx * n * n * sizeof(double);
     double* part           = part_ext;
     if (part_ext)
@@ -778,22 +916,39 @@ int tsgemm(mgx_ctx* ctx, int prec, const double* A, const double* B, int64_t ld,
         MGX_REQUIRE(ctx, per_chunk <= part_cap, "subdivx * n * n * 8 bytes exceed the scratch buffer");
         nchunk = (int)std::min<size_t>((size_t)nchunk, part_cap / per_chunk);
     }
-    const int64_t rows = (lnp + nchunk - 1) / nchunk;
-    if (!part_ext)
+    else
     {
         part = (double*)workspace(ctx, 7, per_chunk * nchunk);
         if (!part) return set_err(ctx, MGX_ENOMEM, "workspace allocation failed");
     }
-    dim3 grid(ntiles, nchunk, subdivx), blk(64 * kWaves);
+    // 16-byte loads where every column of every slab is aligned for them
+    const bool vec = ((((uintptr_t)A | (uintptr_t)B) & 15) | (ld & 1) | (subdivx > 1 ? lnp & 1 : 0)) == 0;
+    const dim3 grid((unsigned)(pairs * nchunk), 1, subdivx), blk(64 * kWaves);
+    auto launch = [&](auto P, auto W) {
+        constexpr int PREC = decltype(P)::value, TW = decltype(W)::value;
+        if (vec)
+            hipLaunchKernelGGL((k_tsgemm<PREC, TW, true>), grid, blk, 0, ctx->stream, A, B, ld, lnp, n, npan, nchunk,
+                lower_only, part);
+        else
+            hipLaunchKernelGGL((k_tsgemm<PREC, TW, false>), grid, blk, 0, ctx->stream, A, B, ld, lnp, n, npan, nchunk,
+                lower_only, part);
+    };
+    auto widths = [&](auto P) {
+        switch (tw)
+        {
+            case 1: launch(P, std::integral_constant<int, 1>()); break;
+            case 2: launch(P, std::integral_constant<int, 2>()); break;
+            case 3: launch(P, std::integral_constant<int, 3>()); break;
+            default: launch(P, std::integral_constant<int, 4>());
+        }
+    };
     if (prec == MGX_PREC_F64)
-        hipLaunchKernelGGL(k_tsgemm<MGX_PREC_F64>, grid, blk, 0, ctx->stream, A, B, ld, lnp, n, ntile, nchunk, rows,
-            lower_only, part);
+        widths(std::integral_constant<int, MGX_PREC_F64>());
     else
-        hipLaunchKernelGGL(k_tsgemm<MGX_PREC_SPLIT>, grid, blk, 0, ctx->stream, A, B, ld, lnp, n, ntile, nchunk,
-            rows, lower_only, part);
+        widths(std::integral_constant<int, MGX_PREC_SPLIT>());
     MGX_CHECK_LAUNCH(ctx);
-    const int64_t tot = (int64_t)n * n * subdivx;
-    hipLaunchKernelGGL(k_chunk_reduce, dim3(nblocks(tot)), dim3(kBlock), 0, ctx->stream, (const double*)part, n,
+    const int64_t nt = ((int64_t)n * n + 31) / 32 * subdivx;
+    hipLaunchKernelGGL(k_chunk_reduce, dim3(nblocks(nt, 1)), dim3(256), 0, ctx->stream, (const double*)part, n,
         nchunk, subdivx, vel, lower_only, ss);
     MGX_CHECK_LAUNCH(ctx);
     return MGX_OK;

@@ -51,6 +51,37 @@ def test_local_gram_and_product_f64(ctx, n, ld, lnp, sub):
     assert relmax(to_np(ts), O.local_product(psi, hp, lnp, sub, vel)) <= 1e-13
 
 
+@pytest.mark.parametrize("prec", [mgx.PREC_F64, mgx.PREC_SPLIT])
+@pytest.mark.parametrize("n,ld,lnp,sub", [(1, 40, 7, 1), (3, 5000, 4999, 1), (16, 640, 320, 2), (17, 301, 100, 3),
+                                          (33, 2048, 2048, 1), (48, 1031, 515, 2), (65, 4100, 4100, 1),
+                                          (97, 777, 777, 1), (130, 600, 299, 2), (255, 1500, 1500, 1)])
+def test_local_products_panels(ctx, prec, n, ld, lnp, sub):
+    """Every panel width (1 to 4 tiles), one to four panels, ragged last tiles
+    and panels, rows not multiples of 16, odd leading dimensions and slab
+    starts (unaligned columns), fewer rows than one chunk.  FP64: 1e-13 of the
+    largest entry as above; split: 2^-24 relative per product, FP32 sums of 16
+    (hi * hi) and 32 (hi * lo) products: 20 * 2^-24 of the sum of |a||b| bounds
+    it, here 1.2e-6 of the largest entry of |A|^T |B|."""
+    rng = np.random.default_rng(n)
+    psi, hp = rng.standard_normal((n, ld)), rng.standard_normal((n, ld))
+    vel = 0.027
+    tp, th = to_dev(psi), to_dev(hp)
+    ts = to_dev(np.full((sub, n, n), np.nan))
+    size = np.max(O.local_product(np.abs(psi), np.abs(hp), lnp, sub, vel))
+    for name, b, args, ref in [("mgx_local_gram", psi, (mgx.ptr(tp),), O.local_gram(psi, lnp, sub, vel)),
+                               ("mgx_local_product", hp, (mgx.ptr(tp), mgx.ptr(th)),
+                                O.local_product(psi, hp, lnp, sub, vel))]:
+        ctx.call(name, prec, *args, ld, lnp, n, sub, vel, mgx.ptr(ts))
+        got = to_np(ts)
+        err = float(np.max(np.abs(got - ref)))
+        if prec == mgx.PREC_F64:
+            assert err <= 1e-13 * np.max(np.abs(ref)) + 1e-14 * size, name
+        else:
+            assert err <= 1.2e-6 * size, name
+        if name == "mgx_local_gram":
+            assert np.array_equal(got, np.transpose(got, (0, 2, 1)))
+
+
 def test_local_gram_split_error(ctx):
     """hi/lo split on FP32 MFMA: error vs FP64 stated and bounded."""
     rng = np.random.default_rng(11)

@@ -38,6 +38,30 @@ def _run(ctx, mg_, rho, vh0, lap_type, **kw):
     return to_np(tvh), st
 
 
+@pytest.mark.parametrize("lap_type,dims,bc,nu,levels", [
+    (0, (44, 20, 100), (1, 1, 1), (2, 2), 10), (2, (36, 72, 40), (1, 1, 1), (2, 2), 10), (1, (2, 64, 6), (1, 1, 1), (2, 2), 10),
+    (0, (16, 40, 68), (0, 1, 0), (2, 2), 10), (2, (20, 12, 132), (0, 0, 0), (2, 2), 10), (0, (5, 7, 9), (1, 1, 1), (2, 2), 10),
+    (0, (32, 32, 32), (1, 1, 1), (2, 2), 1), (0, (32, 32, 32), (1, 1, 1), (2, 2), 0), (0, (64, 64, 64), (1, 1, 1), (2, 2), 10),
+    (0, (24, 24, 24), (1, 1, 1), (3, 1), 10), (2, (24, 24, 24), (1, 1, 1), (1, 2), 10)])
+def test_cycle_shapes_match_oracle(ctx, lap_type, dims, bc, nu, levels):
+    """Tiles with remainders, short and odd directions, one level, one coarse
+    level, coarse levels in one launch and in several, Dirichlet directions,
+    and other sweep counts (the general path)."""
+    og, mg_, rho = _case(lap_type, dims, seed=8, bc=bc)
+    rng = np.random.default_rng(4)
+    vh0 = O.embed(og, 0.1 * rng.standard_normal((1,) + tuple(dims)))
+    got, st = _run(ctx, mg_, rho, vh0, lap_type, max_sweeps=3, tol=0.0, nu1=nu[0], nu2=nu[1], max_nlevels=levels)
+    ref = vh0.copy()
+    conv, fin, rel, red, sweeps = O.poisson_mgm(og, lap_type, rho, ref, nu1=nu[0], nu2=nu[1], max_sweeps=3, tol=0.0,
+                                                max_nlevels=levels, bc=bc)
+    err = relmax(O.interior(og, got), O.interior(og, ref))
+    say("poisson", lap_type, dims, bc, nu, levels, err)
+    assert err <= 1e-12
+    assert st.nb_sweeps == 3 and not st.converged
+    assert st.final_residual == pytest.approx(fin, rel=1e-9)
+    assert np.array_equal(O.trade(og, got.copy(), bc), got)
+
+
 @pytest.mark.parametrize("lap_type,dims", [(0, (32, 32, 32)), (1, (16, 24, 32)), (2, (32, 16, 16))])
 def test_fixed_cycles_match_oracle(ctx, lap_type, dims):
     og, mg_, rho = _case(lap_type, dims)

@@ -318,6 +318,143 @@ __global__ void k_tri(double* L, int n, int zero_upper)
     }
 }
 
+// The inverse of a symmetric positive definite block (order m <= 128, its lower
+// triangle read) by symmetric sweeps in registers: pivot k with d = a_kk turns
+// a_ij into a_ij - a_ik a_jk / d, a_ik into a_ik / d and d into -1/d; m sweeps
+// leave minus the inverse.  528 threads each hold a 4 x 4 tile on or below the
+// diagonal; the pivot column goes through LDS (two buffers, one barrier per
+// sweep).  Bound by the sweeps' chain, about 0.5 us each: 62 us at m = 128,
+// where the library's blocked Cholesky and inverse take about 0.5 ms in 50
+// launches.  *info (a double beside the step's scalars): 1 + the first pivot
+// that is not positive, else 0; first: no block came before.
+constexpr int kSpdB = 128;
+__global__ void __launch_bounds__(576) k_spd_sweep(const double* A, int64_t ld, int m, double* P, int ldp, double* info,
+    int k0, int first)
+{
+    __shared__ double v[2][kSpdB];
+    // tile (tr, tc), tc <= tr, of thread t = tr (tr + 1) / 2 + tc
+    const int t = threadIdx.x;
+    int tr      = (int)((sqrtf(8.f * (float)t + 1.f) - 1.f) * 0.5f);
+    while ((tr + 1) * (tr + 2) / 2 <= t)
+        tr++;
+    while (tr * (tr + 1) / 2 > t)
+        tr--;
+    const int tc   = t - tr * (tr + 1) / 2;
+    const bool act = t < kSpdB / 4 * (kSpdB / 4 + 1) / 2 && 4 * tr < m;
+    double a[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+        {
+            // a diagonal tile is held in full
+            const int r = max(4 * tr + i, 4 * tc + j), c = min(4 * tr + i, 4 * tc + j);
+            a[i][j]     = act && r < m ? A[(int64_t)c * ld + r] : (r == c ? 1. : 0.);
+        }
+    double bad = 0.;
+    for (int k4 = 0; 4 * k4 < m; k4++)
+    {
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++)
+        {
+            const int k = 4 * k4 + kk;  // padding pivots (k >= m) are ones
+            double* w   = v[k & 1];
+            if (act)
+            {
+                if (tc == k4)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        w[4 * tr + i] = a[i][kk];
+                else if (tr == k4)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        w[4 * tc + j] = a[kk][j];
+            }
+            __syncthreads();
+            const double d = w[k];
+            if (!(d > 0.) && bad == 0. && k < m) bad = (double)(k0 + k + 1);
+            // 1 / d: the hardware's estimate and two Newton steps, a third of
+            // the division's chain
+            double inv = __builtin_amdgcn_rcp(d);
+            inv        = __builtin_fma(inv, __builtin_fma(-d, inv, 1.), inv);
+            inv        = __builtin_fma(inv, __builtin_fma(-d, inv, 1.), inv);
+            if (!act) continue;
+            double wr[4], wc[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+            {
+                wr[i] = w[4 * tr + i] * inv;
+                wc[i] = w[4 * tc + i];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    a[i][j] = __builtin_fma(-wr[i], wc[j], a[i][j]);
+            // the pivot's row and column, in the tiles that hold them
+            if (tc == k4)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    a[i][kk] = wr[i];
+            if (tr == k4)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    a[kk][j] = wc[j] * inv;
+            if (tr == k4 && tc == k4) a[kk][kk] = -inv;
+        }
+    }
+    if (act)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+            {
+                const int r = 4 * tr + i, c = 4 * tc + j;
+                if (r < m && c <= r)
+                {
+                    P[(int64_t)c * ldp + r] = -a[i][j];
+                    P[(int64_t)r * ldp + c] = -a[i][j];
+                }
+            }
+    if (t == 0 && (first || (*info == 0. && bad != 0.))) *info = bad;
+}
+
+// the block column [k0, k0 + m) of X to Q (n x m), its own rows zero
+__global__ void k_spd_panel(const double* X, int n, int k0, int m, double* Q)
+{
+    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < (int64_t)n * m; t += (int64_t)gridDim.x * blockDim.x)
+    {
+        const int row = (int)(t % n);
+        Q[t]          = row >= k0 && row < k0 + m ? 0. : X[(int64_t)k0 * n + t];
+    }
+}
+
+// and back: block column and row from B = Q P, the block from -P
+__global__ void k_spd_panel_back(double* X, int n, int k0, int m, const double* B, const double* P)
+{
+    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < (int64_t)n * m; t += (int64_t)gridDim.x * blockDim.x)
+    {
+        const int j = (int)(t / n), row = (int)(t - (int64_t)j * n);
+        const bool in = row >= k0 && row < k0 + m;
+        const double b = in ? -P[(int64_t)j * m + row - k0] : B[t];
+        X[(int64_t)(k0 + j) * n + row] = b;
+        if (!in) X[(int64_t)row * n + k0 + j] = b;
+    }
+}
+
+// X <- -X, exactly symmetric (the lower triangle counts)
+__global__ void k_spd_neg(double* X, int n)
+{
+    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < (int64_t)n * n; t += (int64_t)gridDim.x * blockDim.x)
+    {
+        const int col = (int)(t / n), row = (int)(t - (int64_t)col * n);
+        if (row < col) continue;
+        const double v              = -X[t];
+        X[t]                        = v;
+        X[(int64_t)row * n + col] = v;
+    }
+}
+
 // single block: out = sum_{i,k} H(i,k) * Sinv(k,i)
 __global__ void __launch_bounds__(1024) k_trace_prod(const double* H, const double* Sinv, int n, double* out)
 {
@@ -978,6 +1115,68 @@ int chol_inv(mgx_ctx* ctx, int n, const double* S, double* L, double* Sinv)
     return MGX_OK;
 }
 
+// X = S^-1 for a symmetric positive definite S (lower triangle read; X apart
+// from S), without its Cholesky factor: one launch up to order 128, else the
+// same sweeps by blocks of 128 (the block's inverse P, the panel B = Q P, the
+// rank-128 update X - B Q^T as a library product, five launches a block).
+// info (device) receives 1 + the index of the first pivot that is not
+// positive, else 0.  n = 2048: 1.9 ms against the library's 7.3 ms;
+// 512: 0.38 ms against 1.6 ms.
+int spd_inv_launch(mgx_ctx* ctx, int n, const double* S, double* X, double* info)
+{
+    if (n <= kSpdB)
+    {
+        hipLaunchKernelGGL(k_spd_sweep, dim3(1), dim3(576), 0, ctx->stream, S, (int64_t)n, n, X, n, info, 0, 1);
+        MGX_CHECK_LAUNCH(ctx);
+        return MGX_OK;
+    }
+    double* Q = (double*)workspace(ctx, 7, (2 * (size_t)n * kSpdB + (size_t)kSpdB * kSpdB) * sizeof(double));
+    if (!Q) return set_err(ctx, MGX_ENOMEM, "workspace allocation failed");
+    double *B = Q + (size_t)n * kSpdB, *P = B + (size_t)n * kSpdB;
+    const double one = 1., zero = 0., mone = -1.;
+    rocblas_set_pointer_mode(ctx->blas, rocblas_pointer_mode_host);
+    MGX_CHECK_HIP(ctx, hipMemcpyAsync(X, S, (size_t)n * n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
+    hipLaunchKernelGGL(k_tri, dim3(nblocks((int64_t)n * n)), dim3(kBlock), 0, ctx->stream, X, n, 0);
+    for (int k0 = 0; k0 < n; k0 += kSpdB)
+    {
+        const int m = std::min(kSpdB, n - k0);
+        hipLaunchKernelGGL(k_spd_sweep, dim3(1), dim3(576), 0, ctx->stream, (const double*)X + (size_t)k0 * n + k0,
+            (int64_t)n, m, P, m, info, k0, k0 == 0);
+        hipLaunchKernelGGL(k_spd_panel, dim3(nblocks((int64_t)n * m)), dim3(kBlock), 0, ctx->stream, (const double*)X, n,
+            k0, m, Q);
+        MGX_CHECK_LAUNCH(ctx);
+        if (rocblas_dgemm(ctx->blas, rocblas_operation_none, rocblas_operation_none, n, m, m, &one, Q, n, P, m, &zero, B, n)
+                != rocblas_status_success
+            || rocblas_dgemm(ctx->blas, rocblas_operation_none, rocblas_operation_transpose, n, n, m, &mone, B, n, Q, n,
+                   &one, X, n)
+                   != rocblas_status_success)
+            return set_err(ctx, MGX_EHIP, "rocblas_dgemm failed");
+        hipLaunchKernelGGL(k_spd_panel_back, dim3(nblocks((int64_t)n * m)), dim3(kBlock), 0, ctx->stream, X, n, k0, m,
+            (const double*)B, (const double*)P);
+    }
+    hipLaunchKernelGGL(k_spd_neg, dim3(nblocks((int64_t)n * n)), dim3(kBlock), 0, ctx->stream, X, n);
+    MGX_CHECK_LAUNCH(ctx);
+    return MGX_OK;
+}
+
+int spd_check(mgx_ctx* ctx, double info)
+{
+    if (info == 0.) return MGX_OK;
+    return set_err(ctx, MGX_ENOTSPD, "ERROR in GramMatrix<MatrixType>::updateLS(): potrf info != 0");
+}
+
+// spd_inv_launch with its check (waits for the stream)
+int spd_inv(mgx_ctx* ctx, int n, const double* S, double* X)
+{
+    double* info = (double*)workspace(ctx, 6, 64);
+    if (!info) return set_err(ctx, MGX_ENOMEM, "workspace allocation failed");
+    if (int rc = spd_inv_launch(ctx, n, S, X, info)) return rc;
+    double h = 0.;
+    MGX_CHECK_HIP(ctx, hipMemcpyAsync(&h, info, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    MGX_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return spd_check(ctx, h);
+}
+
 int diag_sum(mgx_ctx* ctx, int n, const double* A, double* dev_out)
 {
     hipLaunchKernelGGL(k_diag_sum, dim3(1), dim3(256), 0, ctx->stream, A, n, dev_out);
@@ -985,67 +1184,19 @@ int diag_sum(mgx_ctx* ctx, int n, const double* A, double* dev_out)
     return MGX_OK;
 }
 
-// Refresh X ~ S^-1 by Newton-Schulz steps X <- X (2I - S X) from the previous
-// inverse (S changes little between orbital steps, so the iteration starts
-// well inside its quadratic basin).  Falls back to the Cholesky inverse when
-// max|I - S X| does not start below 0.25 (first step, large change) or fails
-// to contract.  work: 2 n^2 doubles.  *steps = Newton-Schulz steps taken
-// (-1 when the Cholesky path ran).
-int inverse_update(mgx_ctx* ctx, int n, const double* S, double* L, double* X, double* work, int* steps)
-{
-    const double one = 1., zero = 0., mone = -1., two = 2.;
-    const size_t nn = (size_t)n * n;
-    double* T  = work;
-    double* X2 = work + nn;
-    double* bm = (double*)workspace(ctx, 4, 1024 * sizeof(double));
-    if (!bm) return set_err(ctx, MGX_ENOMEM, "workspace allocation failed");
-    rocblas_set_pointer_mode(ctx->blas, rocblas_pointer_mode_host);
-    double prev = 1e300;
-    *steps      = 0;
-    for (int it = 0; it < 8; it++)
-    {
-        if (rocblas_dgemm(ctx->blas, rocblas_operation_none, rocblas_operation_none, n, n, n, &one, S, n, X, n, &zero,
-                T, n)
-            != rocblas_status_success)
-            return set_err(ctx, MGX_EHIP, "rocblas_dgemm failed");
-        const int nb = 512;
-        hipLaunchKernelGGL(k_id_err, dim3(nb), dim3(256), 0, ctx->stream, (const double*)T, n, bm);
-        hipLaunchKernelGGL(k_max_reduce, dim3(1), dim3(256), 0, ctx->stream, (const double*)bm, nb, bm + nb);
-        MGX_CHECK_LAUNCH(ctx);
-        double delta = 0.;
-        MGX_CHECK_HIP(ctx, hipMemcpyAsync(&delta, bm + nb, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        MGX_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (!(delta < 0.25) || delta > 0.5 * prev)
-        {
-            *steps = -1;
-            return chol_inv(ctx, n, S, L, X);
-        }
-        if (delta < 1e-15) break;
-        // X2 = 2 X - X T
-        MGX_CHECK_HIP(ctx, hipMemcpyAsync(X2, X, nn * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-        if (rocblas_dgemm(ctx->blas, rocblas_operation_none, rocblas_operation_none, n, n, n, &mone, X, n, T, n, &two,
-                X2, n)
-            != rocblas_status_success)
-            return set_err(ctx, MGX_EHIP, "rocblas_dgemm failed");
-        MGX_CHECK_HIP(ctx, hipMemcpyAsync(X, X2, nn * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-        (*steps)++;
-        prev = delta;
-        if (delta < 3e-8) break;  // the error after this step is ~delta^2
-    }
-    hipLaunchKernelGGL(k_symmetrize, dim3(nblocks((int64_t)nn)), dim3(kBlock), 0, ctx->stream, X, n);
-    MGX_CHECK_LAUNCH(ctx);
-    return MGX_OK;
-}
-
-// inverse_update for a pair-sparse S (values Sv per pair, column tiles pt):
+// Refresh X ~ S^-1 by Newton-Schulz steps from the previous inverse (S changes
+// little between orbital steps, so the iteration starts well inside its
+// quadratic basin), S pair-sparse (values Sv per pair, column tiles pt):
 // T = X S on the sparse product, X <- 2X - T X as one dense GEMM (written to
 // the other half of the work buffer, operands swapped, no copies).  Stops
 // before a step once delta = max|I - X S| < tol.  With FP64 products it also
 // stops after a step once delta^2 (the error that step leaves) < tol; with
 // lowp the correction E X, E = I - X S, is one FP32 product, whose rounding
 // (~1e-7 |E| |X|) can exceed delta^2, so only measured deltas end the loop.
-int inverse_update_pairs(mgx_ctx* ctx, int n, const double* S, const double* Sv, const PairTiles& pt, double* L,
-    double* X, double* work, int* steps, double tol, bool lowp)
+// Falls back to spd_inv when delta does not start below 0.25 (a large change)
+// or fails to contract; *steps = steps taken (-1: spd_inv ran).  work: 2 n^2.
+int inverse_update_pairs(mgx_ctx* ctx, int n, const double* S, const double* Sv, const PairTiles& pt, double* X,
+    double* work, int* steps, double tol, bool lowp)
 {
     const double mone = -1., two = 2.;
     const size_t nn = (size_t)n * n;
@@ -1084,7 +1235,7 @@ int inverse_update_pairs(mgx_ctx* ctx, int n, const double* S, const double* Sv,
         if (!(delta < 0.25) || delta > 0.5 * prev)
         {
             *steps = -1;
-            return chol_inv(ctx, n, S, L, X);
+            return spd_inv(ctx, n, S, X);
         }
         if (delta < tol) break;
         if (lowp)
@@ -1418,7 +1569,9 @@ int mgx_mehr_projected(mgx_ctx* ctx, int n, const double* S, const double* Sinv,
     double* w       = (double*)workspace(ctx, 5, 2 * nn * sizeof(double) + 64);
     if (!w) return set_err(ctx, MGX_ENOMEM, "workspace allocation failed");
     // invB (ProjectedMatricesMehrstellen::computeInvB: potrf + potri)
-    int rc = chol_inv(ctx, n, B, w, invB);
+    if (invB == B)
+        MGX_CHECK_HIP(ctx, hipMemcpyAsync(w, B, nn * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
+    int rc = spd_inv(ctx, n, invB == B ? w : B, invB);
     if (rc) return rc;
     // theta = invB H (updateTheta)
     if ((rc = mgx::theta(ctx, n, invB, H, theta))) return rc;

@@ -4,7 +4,7 @@
 //
 //   hpsi = H psi                        Hamiltonian::applyLocal
 //   S, H = psi^T psi, psi^T H psi       computeGram / addHlocalij
-//   L, S^-1 = chol / inverse            GramMatrix::updateLS / computeInverse
+//   S^-1                                GramMatrix::updateLS / computeInverse
 //   theta = S^-1 H, E = tr(H S^-1)      updateTheta / getEigSum
 //   R = psi theta - hpsi, |R|           computeResidualUsingHPhi / ConstraintResidual
 //   stop if |R| < tol                   ABPG::updateWF early return
@@ -27,8 +27,8 @@ int box_hloc(mgx_ctx*, const mgx_boxset*, int, const void*, const double*, void*
 int box_gram_h(mgx_ctx*, const mgx_boxset*, int, const double*, const double*, double*, double*, double*, double*);
 PairTiles boxset_tiles(const mgx_boxset*);
 int64_t boxset_npairs(const mgx_boxset*);
-int inverse_update_pairs(mgx_ctx*, int, const double*, const double*, const PairTiles&, double*, double*, double*,
-    int*, double, bool);
+int inverse_update_pairs(mgx_ctx*, int, const double*, const double*, const PairTiles&, double*, double*, int*,
+    double, bool);
 int box_residual(mgx_ctx*, const mgx_boxset*, const double*, const double*, const double*, double*, double*);
 int box_sumsq(mgx_ctx*, const mgx_boxset*, const double*, double*);
 int box_norm(mgx_ctx*, const mgx_boxset*, const double*, const double*, double*);
@@ -41,11 +41,12 @@ int box_residual_start(mgx_ctx*, const mgx_boxset*, const double*, const double*
 bool boxset_has_cells(const mgx_boxset*);
 int64_t box_size(const mgx_boxset*, int);
 void boxset_geom(const mgx_boxset*, int gdim[3], double h[3], int* nbox);
-int chol_inv(mgx_ctx*, int, const double*, double*, double*);
+int spd_inv_launch(mgx_ctx*, int, const double*, double*, double*);
+int spd_check(mgx_ctx*, double);
+int spd_inv(mgx_ctx*, int, const double*, double*);
 int theta(mgx_ctx*, int, const double*, const double*, double*);
 int trace_prod(mgx_ctx*, int, const double*, const double*, double*);
 int diag_sum(mgx_ctx*, int, const double*, double*);
-int inverse_update(mgx_ctx*, int, const double*, double*, double*, double*, int*);
 int ritz(mgx_ctx*, int, const double*, const double*, double*, double*);
 int box_anderson_dots(mgx_ctx*, const mgx_boxset*, int, const void*, double, const void*, const double*, double*,
     double*);
@@ -103,7 +104,7 @@ struct mgx_solver
     int iter       = 0;
     double *psi = nullptr, *psi0 = nullptr, *hpsi = nullptr, *res = nullptr, *vtot = nullptr;
     MgxProf prof;
-    double *S = nullptr, *H = nullptr, *L = nullptr, *Sinv = nullptr, *th = nullptr;
+    double *S = nullptr, *H = nullptr, *Sinv = nullptr, *th = nullptr;
     double *eig = nullptr, *d = nullptr, *scal = nullptr, *nswork = nullptr;
     double *Sv = nullptr, *Hv = nullptr;  // S, H per interacting pair
     // Mehrstellen: B psi, the B-matrix and its inverse
@@ -168,7 +169,7 @@ namespace
 
 void free_solver(mgx_solver* s)
 {
-    double* bufs[] = { s->psi, s->psi0, s->hpsi, s->res, s->vtot, s->S, s->H, s->L, s->Sinv, s->th, s->eig, s->d,
+    double* bufs[] = { s->psi, s->psi0, s->hpsi, s->res, s->vtot, s->S, s->H, s->Sinv, s->th, s->eig, s->d,
         s->scal, s->nswork, s->Sv, s->Hv, s->x0, s->psi_prev, s->r_prev, s->psi_cnn, s->r_cnn, s->bpsi, s->Bm,
         s->invB, s->xprev };
     for (double* b : bufs)
@@ -240,7 +241,8 @@ int head_body(mgx_solver* s, bool pending, bool chol, int spec, bool bf16)
     // the Newton-Schulz refresh from the previous inverse
     if (chol)
     {
-        if ((rc = chol_inv(ctx, s->n, s->S, s->L, s->Sinv))) return rc;
+        // whether S was positive definite comes with the step's scalars
+        if ((rc = spd_inv_launch(ctx, s->n, s->S, s->Sinv, s->scal + 6))) return rc;
     }
     else if ((rc = inverse_update_spec(ctx, s->n, s->Sv, s->tiles, s->Sinv, s->nswork, spec, bf16, s->scal + 8,
                   bf16 ? nullptr : s->xprev, s->have_xprev)))
@@ -374,8 +376,8 @@ int head_mehr(mgx_solver* s, bool pending)
     if ((rc = box_gram_hb_mehr(ctx, s->bs, s->psi, s->hpsi, s->bpsi, s->vtot, s->S, s->H, s->Bm))) return rc;
     prof_end(ctx, tk);
     tk = prof_begin(ctx, MGX_PROF_DENSE);
-    if ((rc = chol_inv(ctx, s->n, s->S, s->L, s->Sinv))) return rc;
-    if ((rc = chol_inv(ctx, s->n, s->Bm, s->L, s->invB))) return rc;
+    if ((rc = spd_inv_launch(ctx, s->n, s->S, s->Sinv, s->scal + 6))) return rc;
+    if ((rc = spd_inv_launch(ctx, s->n, s->Bm, s->invB, s->scal + 7))) return rc;
     if ((rc = theta(ctx, s->n, s->invB, s->H, s->th))) return rc;
     if ((rc = diag_sum(ctx, s->n, s->th, s->scal))) return rc;
     prof_end(ctx, tk);
@@ -470,7 +472,7 @@ int step_body(mgx_solver* s, double tol, mgx_solver_stats_t* st, bool* done)
     if (mehr)
         rc = head_mehr(s, pending);  // Cholesky of S and of the B-matrix every step
     else if (chol)
-        rc = head_body(s, pending, true, 0, bf16);  // waits for potrf's info: never captured
+        rc = head_body(s, pending, true, 0, bf16);  // the first step and restarts: never captured
     else
     {
         uint64_t key = 1;
@@ -481,6 +483,8 @@ int step_body(mgx_solver* s, double tol, mgx_solver_stats_t* st, bool* done)
     }
     if (rc) return rc;
     MGX_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (chol && (rc = spd_check(ctx, s->host[6]))) return rc;
+    if (mehr && (rc = spd_check(ctx, s->host[7]))) return rc;
     s->pending_norm = false;
     if (chol)
     {
@@ -509,10 +513,10 @@ int step_body(mgx_solver* s, double tol, mgx_solver_stats_t* st, bool* done)
             int steps = 0;
             if (more < 0)
             {
-                if ((rc = chol_inv(ctx, n, s->S, s->L, s->Sinv))) return rc;
+                if ((rc = spd_inv(ctx, n, s->S, s->Sinv))) return rc;
                 steps = -1;
             }
-            else if ((rc = inverse_update_pairs(ctx, n, s->S, s->Sv, s->tiles, s->L, s->Sinv, s->nswork, &steps,
+            else if ((rc = inverse_update_pairs(ctx, n, s->S, s->Sv, s->tiles, s->Sinv, s->nswork, &steps,
                           ns_tol, bf16)))
                 return rc;
             s->ns_steps += spec + std::max(steps, 0);
@@ -746,7 +750,7 @@ int mgx_solver_create(mgx_ctx* ctx, const mgx_boxset* bs, const mgx_solver_cfg_t
     auto alloc = [&](double** p, size_t cnt) { return hipMalloc((void**)p, cnt * sizeof(double)) == hipSuccess; };
     const size_t tsize = cfg->precond_dtype == MGX_F64 ? sizeof(double) : sizeof(float);
     bool ok = alloc(&s->psi, s->npts) && alloc(&s->psi0, s->npts) && alloc(&s->hpsi, s->npts) && alloc(&s->res, s->npts) && alloc(&s->vtot, gsize)
-              && alloc(&s->S, nn) && alloc(&s->H, nn) && alloc(&s->L, nn) && alloc(&s->Sinv, nn) && alloc(&s->th, nn)
+              && alloc(&s->S, nn) && alloc(&s->H, nn) && alloc(&s->Sinv, nn) && alloc(&s->th, nn)
               && alloc(&s->eig, s->n) && alloc(&s->d, 2 * (size_t)s->n + 8) && alloc(&s->scal, 32) && alloc(&s->nswork, 2 * nn)
               && alloc(&s->Sv, (size_t)std::max<int64_t>(boxset_npairs(bs), 1))
               && alloc(&s->Hv, (size_t)std::max<int64_t>(boxset_npairs(bs), 1))
@@ -974,7 +978,7 @@ int mgx_solver_density(mgx_solver* s, double nel, double* rho, double* charge)
     // S of the current psi (FP64; H is a by-product here), its inverse, and
     // dm = 2 S^-1 in theta's buffer
     if ((rc = box_gram_h(ctx, s->bs, MGX_PREC_F64, s->psi, s->psi, s->S, s->H, s->Sv, s->Hv))) return rc;
-    if ((rc = chol_inv(ctx, s->n, s->S, s->L, s->Sinv))) return rc;
+    if ((rc = spd_inv(ctx, s->n, s->S, s->Sinv))) return rc;
     s->have_inv      = true;
     s->have_xprev    = false;
     const int64_t nn = (int64_t)s->n * s->n;

@@ -227,3 +227,41 @@ def test_synth_separable_against_oracle_operator(ctx):
     assert relmax(to_np(th), hs) <= 1e-12
     # normalised over the full grid
     assert np.allclose(h ** 3 * np.sum(full * full, axis=(1, 2, 3)), 1.0, rtol=1e-12)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 24, 64, 127, 128, 129, 131, 200, 256, 300, 513])
+def test_spd_inverse_orders(ctx, n):
+    """The inverse without its factor (through mgx_mehr_projected): tiles of 4
+    with remainders, one block and several, a last block of one and of a few,
+    only the lower triangle read, in place and apart.  Backward stable sweeps:
+    n * cond * 2^-53 of the largest entry, cond(B) < 20 here, with 4 to spare."""
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((n, 2 * n + 4))
+    B = A @ A.T / (2 * n + 4) + 0.2 * np.eye(n)
+    H = rng.standard_normal((n, n))
+    ref = np.linalg.inv(B)
+    junk = np.triu(np.full((n, n), np.nan), 1)  # column-major: numpy's lower triangle is the upper one
+    tB = to_dev((np.tril(B) + junk).T.copy())
+    tS, tI, tH = to_dev(B), to_dev(np.eye(n)), to_dev(H.T.copy())
+    inv, th, hb = to_dev(np.zeros((n, n))), to_dev(np.zeros((n, n))), to_dev(np.zeros((n, n)))
+    args = (mgx.ptr(tH), mgx.ptr(inv), mgx.ptr(th), mgx.ptr(hb), None)
+    ctx.call("mgx_mehr_projected", n, mgx.ptr(tS), mgx.ptr(tI), mgx.ptr(tB), *args)
+    got = to_np(inv)
+    tol = 4 * n * 20 * 2.0 ** -53
+    assert relmax(got, ref) <= tol
+    assert np.array_equal(got, got.T)
+    assert relmax(to_np(th).T, ref @ H) <= 1e-12
+    tB = to_dev(B)
+    ctx.call("mgx_mehr_projected", n, mgx.ptr(tS), mgx.ptr(tI), mgx.ptr(tB), mgx.ptr(tH), mgx.ptr(tB), mgx.ptr(th),
+             mgx.ptr(hb), None)
+    assert np.array_equal(to_np(tB), got)
+
+
+@pytest.mark.parametrize("n,k", [(1, 0), (30, 29), (128, 64), (200, 3), (200, 190)])
+def test_spd_inverse_rejects_indefinite(ctx, n, k):
+    B = 2.0 * np.eye(n)
+    B[k, k] = -1.0
+    t = [to_dev(x) for x in (B, np.eye(n), B, B)]
+    o = [to_dev(np.zeros((n, n))) for _ in range(3)]
+    rc = mgx.lib().mgx_mehr_projected(ctx.h, n, *[mgx.ptr(x) for x in t + o], None)
+    assert rc == mgx.MGX_ENOTSPD

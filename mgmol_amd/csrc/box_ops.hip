@@ -1086,6 +1086,284 @@ __global__ void k_first_sweep(const double* res, T* f, T* x, int64_t n, double j
     }
 }
 
+// ---------------------------------------------------------------------------
+// The levels below the fine one of a box's V-cycle, whole, from LDS.
+//
+// A coarse level of one box is at most a few thousand points, so swept level
+// by level over all boxes the cycle is a chain of launches (two sweeps, the
+// restriction, the prolongation and two sweeps a level, four at the last)
+// that each run for about as long as they take to start.  Here one block per
+// box does all of them: the right hand side is read once and the correction
+// written once.
+//
+// A level's x lies in LDS with one zero element before each row, one zero row
+// before each plane, a zero plane on either side and a last zero row, so that
+// every neighbour outside the box reads the zero it stands for without a
+// test.  On the top level a thread has K points in a row along x: f, x and
+// the neighbours in x stay in registers, and a point costs four LDS reads
+// instead of eight.  Below it, with an eighth of the points, it is one point
+// per thread and f lies in LDS too.  The arithmetic per point is that of
+// k_first_sweep, k_box_jacobi, k_box_restrict2 and k_box_prolong8.
+//
+// Measured, all coarse levels of one cycle: 2048 boxes of edge 32 (top edge
+// 16, FP32) 115 us in 11 launches, 57 in this one (92 with f and every
+// neighbour from LDS); 512 boxes of 24 to 40 (FP64) 132 -> 92; 128 of 20 and
+// 24 (FP64) 70 -> 8; 24 of 8 to 16 (FP32) 40 -> 5.  Left at the top: FP64
+// adds and multiplies and the LDS reads of y and z; one block of 1024 threads
+// per CU at top edge 20, whose FP64 columns spill (f and x from LDS instead:
+// 148 us).
+constexpr int kCoarseLevels = 8;
+constexpr int kCoarseLds    = 160 * 1024;
+
+struct CoarseArgs
+{
+    const int64_t* off;  // offsets per box at the top of these levels
+    const int* edge;
+    const int* order;
+    int shift, nbox, nl;
+    double jf[kCoarseLevels];
+    Coef2 c2[kCoarseLevels];
+};
+
+__host__ __device__ inline int coarse_x_size(int e) { return ((e + 2) * (e + 1) + 1) * (e + 1) + 1; }
+
+// elements from a level's x that a column of K points may read: the planes of
+// whole columns, the margin and the row and element after them
+__host__ __device__ inline int coarse_span(int e, int K)
+{
+    return (((e + K - 1) / K * K + 2) * (e + 1) + 2) * (e + 1) + 1;
+}
+
+// elements of LDS for nl levels from edge e: x of each, f below the top
+__host__ __device__ inline int coarse_lds(int e, int nl)
+{
+    int n = coarse_x_size(e);
+    for (int l = 1; l < nl; l++)
+        n += coarse_x_size(e >> l) + (e >> l) * (e >> l) * (e >> l);
+    return n;
+}
+
+template <typename T>
+__device__ __forceinline__ T coarse_axpy(T x, double s, T y)
+{
+    x += static_cast<T>(s * static_cast<double>(y));
+    return x;
+}
+
+// w of a level of edge e (in X) restricted to Fc
+template <typename T>
+__device__ __forceinline__ void coarse_restrict(const T* X, int e, T* Fc)
+{
+    const int ec = e >> 1, sy = e + 1, sx = sy * sy;
+    const float r2 = 1.f / (float)(ec * ec), r1 = 1.f / (float)ec;
+    for (int p = threadIdx.x; p < ec * ec * ec; p += blockDim.x)
+    {
+        // exact: p + 1/2 stays half a unit off every multiple (p < 2^13)
+        const int x = (int)(((float)p + .5f) * r2);
+        const int q = p - x * ec * ec;
+        const int y = (int)(((float)q + .5f) * r1);
+        const T* u  = X + 1 + (2 * x + 1) * sx + (2 * y + 1) * sy + 2 * (q - y * ec);
+#define F3(dx, dy, dz) (double)u[(dx) * sx + (dy) * sy + (dz)]
+        double face   = F3(1, 0, 0) + F3(-1, 0, 0) + F3(0, 1, 0) + F3(0, -1, 0) + F3(0, 0, -1) + F3(0, 0, 1);
+        // not all 27 loads at once: the registers hold the column's f and x too
+        __builtin_amdgcn_sched_barrier(0);
+        double corner = F3(1, 1, -1) + F3(1, 1, 1) + F3(1, -1, -1) + F3(1, -1, 1) + F3(-1, 1, -1) + F3(-1, 1, 1)
+                        + F3(-1, -1, -1) + F3(-1, -1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        double edge = F3(0, 1, -1) + F3(0, 1, 1) + F3(0, -1, -1) + F3(0, -1, 1) + F3(1, 0, -1) + F3(1, 0, 1)
+                      + F3(-1, 0, -1) + F3(-1, 0, 1) + F3(-1, -1, 0) + F3(1, -1, 0) + F3(-1, 1, 0) + F3(1, 1, 0);
+        Fc[p] = (T)(kInv64 * (8. * F3(0, 0, 0) + 4. * face + 2. * edge + corner));
+#undef F3
+    }
+}
+
+// K points in a row along x, from (x0, y, z), of a box of edge e.  With K = 1
+// every point of the level has its thread.
+template <typename T, int K>
+struct CoarseCol
+{
+    T* X;  // padded x
+    int e, sy, sx;
+    int x0, y, z, i0, km;
+    bool on;  // false: no points; point 0's column is read, nothing written
+    T f[K], x[K];
+
+    __device__ __forceinline__ CoarseCol(T* lds, int edge) : X(lds), e(edge)
+    {
+        sy = e + 1, sx = sy * sy;
+        const int e2 = e * e, t = threadIdx.x;
+        const int sg = (int)(((float)t + .5f) * (1.f / (float)e2));
+        on           = sg * K < e;
+        x0           = on ? sg * K : 0;
+        const int q  = on ? t - sg * e2 : 0;
+        y            = (int)(((float)q + .5f) * (1.f / (float)e));
+        z            = q - y * e;
+        i0           = 1 + (x0 + 1) * sx + (y + 1) * sy + z;
+        km           = e - 1 - x0;
+    }
+    __device__ __forceinline__ bool act(int k) const { return on && k <= km; }
+    // offset of point k in f
+    __device__ __forceinline__ int pf(int k) const { return ((x0 + k) * e + y) * e + z; }
+    __device__ __forceinline__ void load(const T* src)
+    {
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            f[k] = k <= km ? src[pf(k)] : (T)0;
+    }
+    // w = A x - f, zero beyond the box (planes read there lie within the LDS,
+    // coarse_span; a clamped index per point would cost its register)
+    __device__ __forceinline__ void stale(const Coef2& c, T (&w)[K]) const
+    {
+        const T xm = X[i0 - sx], xp = X[i0 + K * sx];
+#pragma unroll
+        for (int k = 0; k < K; k++)
+        {
+            const T* u     = X + i0 + k * sx;
+            const T a      = k > 0 ? x[k > 0 ? k - 1 : 0] : xm;
+            const T b      = k < K - 1 ? x[k < K - 1 ? k + 1 : k] : xp;
+            const double r = c.c0 * x[k] + c.c1x * (T)(a + b) + c.c1y * (T)(u[-sy] + u[sy])
+                             + c.c1z * (T)(u[-1] + u[1]);
+            w[k] = (T)r;
+            w[k] += static_cast<T>(-1. * static_cast<double>(f[k]));
+            if (k > km) w[k] = (T)0;
+        }
+    }
+    __device__ __forceinline__ void store(const T (&v)[K]) const
+    {
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            if (act(k)) X[i0 + k * sx] = v[k];
+    }
+    // x += -jf w; in LDS too, for the next sweep, where it is asked for
+    __device__ __forceinline__ void sweep(const Coef2& c, double jf, bool keep)
+    {
+        T w[K];
+        stale(c, w);
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            x[k] = coarse_axpy(x[k], -1. * jf, w[k]);
+        if (!keep) return;
+        __syncthreads();
+        store(x);
+        __syncthreads();
+    }
+    __device__ __forceinline__ void start(double jf)
+    {
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            x[k] = coarse_axpy((T)0, jf, f[k]);
+        store(x);
+        __syncthreads();
+    }
+    // the second sweep, with its stale residual in LDS for the restriction
+    __device__ __forceinline__ void down(const Coef2& c, double jf)
+    {
+        T w[K];
+        stale(c, w);
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            x[k] = coarse_axpy(x[k], -1. * jf, w[k]);
+        __syncthreads();
+        store(w);
+        __syncthreads();
+    }
+    // x -= P(xc)
+    __device__ __forceinline__ void correct(const T* xc)
+    {
+        const int cy = (e >> 1) + 1, cx = cy * cy, px = x0 >> 1;
+        const T* u = xc + 1 + ((y >> 1) + 1) * cy + (z >> 1);
+        T cc[2][2][2];
+#pragma unroll
+        for (int k = 0; k < K; k++)
+        {
+            if ((k & 1) == 0)
+#pragma unroll
+                for (int a = 0; a < 2; a++)
+                {
+                    const T* v = u + (px + k / 2 + a + 1) * cx;
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        cc[a][q >> 1][q & 1] = v[(q >> 1) * cy + (q & 1)];
+                }
+            const T p = prolong8_val(cc, K == 1 ? x0 & 1 : k & 1, y & 1, z & 1);
+            if (k <= km) x[k] = coarse_axpy(x[k], -1., p);
+        }
+        store(x);
+        __syncthreads();
+    }
+};
+
+// K points per thread on the top level
+template <typename T, int K>
+__global__ void __launch_bounds__(1024) k_box_coarse(const T* __restrict__ f, T* __restrict__ out, CoarseArgs a)
+{
+    static_assert(K % 2 == 0, "a column starts on an even plane");
+    extern __shared__ unsigned char lds_raw[];
+    T* X0           = reinterpret_cast<T*>(lds_raw);
+    const int64_t L = xcd_block(blockIdx.x, gridDim.x);
+    if (L >= a.nbox) return;
+    const int j  = a.order[L];
+    const int e0 = a.edge[j] >> a.shift;
+    const int64_t base = a.off[j];
+    CoarseCol<T, K> top(X0, e0);
+    top.load(f + base);
+    for (int t = threadIdx.x; t < coarse_lds(e0, a.nl); t += blockDim.x)
+        X0[t] = (T)0;
+    __syncthreads();
+    top.start(a.jf[0]);
+    if (a.nl == 1)
+    {
+        for (int it = 1; it < 4; it++)
+            top.sweep(a.c2[0], a.jf[0], it < 3);
+    }
+    else
+    {
+        top.down(a.c2[0], a.jf[0]);
+        T* X = X0 + coarse_x_size(e0);
+        coarse_restrict(X0, e0, X + coarse_x_size(e0 >> 1));
+        for (int l = 1; l < a.nl; l++)
+        {
+            const int e = e0 >> l;
+            T* F        = X + coarse_x_size(e);
+            // f written by other threads of this block (coarse_restrict)
+            __syncthreads();
+            CoarseCol<T, 1> lv(X, e);
+            lv.load(F);
+            lv.start(a.jf[l]);
+            if (l == a.nl - 1)
+            {
+                for (int it = 1; it < 4; it++)
+                    lv.sweep(a.c2[l], a.jf[l], true);
+                break;
+            }
+            lv.down(a.c2[l], a.jf[l]);
+            T* Xc = F + e * e * e;
+            coarse_restrict(X, e, Xc + coarse_x_size(e >> 1));
+            X = Xc;
+        }
+        for (int l = a.nl - 2; l >= 1; l--)
+        {
+            const int e = e0 >> l;
+            const T* Xc = X;
+            X -= coarse_x_size(e) + e * e * e;
+            // x after the second sweep, from f and its stale residual w
+            CoarseCol<T, 1> lv(X, e);
+            lv.load(X + coarse_x_size(e));
+            lv.x[0] = coarse_axpy(coarse_axpy((T)0, a.jf[l], lv.f[0]), -1. * a.jf[l], X[lv.i0]);
+            __syncthreads();
+            lv.correct(Xc);
+            lv.sweep(a.c2[l], a.jf[l], true);
+            lv.sweep(a.c2[l], a.jf[l], true);
+        }
+        top.correct(X);
+        top.sweep(a.c2[0], a.jf[0], true);
+        top.sweep(a.c2[0], a.jf[0], false);
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++)
+        if (top.act(k)) out[base + top.pf(k)] = top.x[k];
+}
+
 // per-box scale of the residual for the FP16 V-cycle: sc_j brings the box's
 // RMS of R to kF16Rms (FP16 keeps 11 bits between 6e-5 and 65504; the
 // V-cycle is linear, so its FP32 output is divided by sc_j); inv_j = 1/sc_j.
@@ -3312,6 +3590,54 @@ int box_mg_setup(mgx_ctx* ctx, const mgx_boxset* bs, int max_levels, BoxMG<T>& B
     return MGX_OK;
 }
 
+// The levels from `level` on (the coarse ones: 2nd order operator, zero start,
+// the iterate of `level` to out) by k_box_coarse; false where a box's levels
+// do not fit its LDS or a thread's points its registers.  FP32 and FP64 only:
+// the FP16 cycle rounds its FP32 arithmetic at other places.
+template <typename T>
+bool box_coarse(mgx_ctx* ctx, const mgx_boxset* bs, int level, int max_levels, const T* f, T* out, int* rc, bool run)
+{
+    if constexpr (sizeof(T) < 4) return false;
+    else
+    {
+        CoarseArgs a;
+        a.nl = max_levels - level + 1;
+        const int e = bs->maxedge >> level;
+        if (a.nl > kCoarseLevels || e > 20) return false;
+        // short columns while the block is not full (edge 12, 128 boxes: 8.3 us
+        // with 2, 9 with 4, 33 with 8 points at once); a block of 1024 at most
+        // beyond (edge 16, 2048 boxes, FP32: 78 us with 4 points, 57 with 8)
+        const int K = e <= 12 ? 2 : e <= 16 ? 8 : 10;
+        // every term grows with the edge: the largest box's are enough
+        const int elems    = std::max({ coarse_lds(e, a.nl), coarse_span(e, K),
+            a.nl > 1 ? coarse_x_size(e) + coarse_span(e / 2, K / 2) : 0 });
+        const size_t bytes = sizeof(T) * (size_t)elems;
+        if (bytes > (size_t)kCoarseLds) return false;
+        if (!run) return true;
+        for (int l = 0; l < a.nl; l++)
+        {
+            const double s    = (double)((int64_t)1 << (level + l));
+            const double h[3] = { bs->h[0] * s, bs->h[1] * s, bs->h[2] * s };
+            a.jf[l]           = jacobi_factor(MGX_LAP_2ND, h);
+            a.c2[l]           = coef2(h);
+        }
+        a.off = bs->d_off[level], a.edge = bs->d_edge, a.order = bs->d_sp_col;
+        a.shift = level, a.nbox = bs->nbox;
+        const int nt      = std::max(e * e * ((e + K - 1) / K), a.nl > 1 ? (e / 2) * (e / 2) * (e / 2) : 0);
+        const int NT      = (nt + 63) / 64 * 64;
+        const auto kernel = K == 2 ? k_box_coarse<T, 2> : K == 8 ? k_box_coarse<T, 8> : k_box_coarse<T, 10>;
+        if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes)
+            != hipSuccess)
+        {
+            *rc = set_err(ctx, MGX_EHIP, "k_box_coarse: LDS size");
+            return true;
+        }
+        hipLaunchKernelGGL(kernel, dim3((bs->nbox + 7) / 8 * 8), dim3(NT), bytes, ctx->stream, f, out, a);
+        *rc = MGX_OK;
+        return true;
+    }
+}
+
 // Preconditioning<T>::mg, src/Preconditioning.cc:155-216, masks implicit.
 // Sweeps ping-pong between v and tmp; every sweep count is even, so the
 // result is back in v.
@@ -3338,6 +3664,10 @@ int box_mg_rec(mgx_ctx* ctx, const mgx_boxset* bs, BoxMG<T>& B, int max_levels, 
     // restricts it itself (MGX_TUNE_RESTRICT choice 1, where it applies)
     T* rcoarse    = level < max_levels ? B.rc[level] : nullptr;
     bool restricted = false;
+    // the levels below by one launch from LDS, where they fit: then no start
+    // is written for them
+    const bool lds_below = level < max_levels
+                           && box_coarse<T>(ctx, bs, level + 1, max_levels, nullptr, nullptr, nullptr, false);
     for (int it = first_done ? 1 : 0; it < ncycl; it++)
     {
         T* w          = (it == ncycl - 1 && level < max_levels) ? B.w[level] : nullptr;
@@ -3345,12 +3675,12 @@ int box_mg_rec(mgx_ctx* ctx, const mgx_boxset* bs, BoxMG<T>& B, int max_levels, 
         const int tok = level == 0 ? prof_begin(ctx, MGX_PROF_JACOBI0, (w ? 4. : 3.) * st * np0) : -1;
         // fused, the coarse level's zero-start first sweep is written too
         if ((rc = box_jacobi_t(ctx, bs, level, type, jf, (const T*)a, f, b, w, nullptr, nullptr, rfuse,
-                 &restricted, (const T*)nullptr, rfuse ? B.tmp[level + 1] : (T*)nullptr,
+                 &restricted, (const T*)nullptr, rfuse && !lds_below ? B.tmp[level + 1] : (T*)nullptr,
                  jacobi_factor(MGX_LAP_2ND, hc))))
             return rc;
         prof_end(ctx, tok);
         // fused: x and f read, x written, the coarse residual and start written
-        if (restricted) prof_retag(ctx, tok, MGX_PROF_JACOBI0, (3. + 2. / 8.) * st * np0);
+        if (restricted) prof_retag(ctx, tok, MGX_PROF_JACOBI0, (3. + (lds_below ? 1. : 2.) / 8.) * st * np0);
         std::swap(a, b);
     }
     if (level == max_levels) return MGX_OK;
@@ -3364,14 +3694,22 @@ int box_mg_rec(mgx_ctx* ctx, const mgx_boxset* bs, BoxMG<T>& B, int max_levels, 
     }
     // the coarse level starts from 0: its first sweep is pointwise (written
     // by the fused restriction, else here)
-    if (!restricted)
+    if (lds_below)
+    {
+        box_coarse<T>(ctx, bs, level + 1, max_levels, (const T*)rcoarse, nv, &rc, true);
+        if (rc) return rc;
+        MGX_CHECK_LAUNCH(ctx);
+    }
+    else if (!restricted)
     {
         const int64_t nc = bs->off[level + 1][bs->nbox];
         hipLaunchKernelGGL(k_first_sweep<T>, dim3(nblocks(nc)), dim3(kBlock), 0, ctx->stream,
             (const double*)nullptr, rcoarse, B.tmp[level + 1], nc, jacobi_factor(MGX_LAP_2ND, hc));
         MGX_CHECK_LAUNCH(ctx);
     }
-    if ((rc = box_mg_rec(ctx, bs, B, max_levels, nv, (const T*)rcoarse, MGX_LAP_2ND, level + 1, true))) return rc;
+    if (!lds_below
+        && (rc = box_mg_rec(ctx, bs, B, max_levels, nv, (const T*)rcoarse, MGX_LAP_2ND, level + 1, true)))
+        return rc;
     // the coarse correction prolonged inside the first post-sweep
     // (MGX_TUNE_PROLONG choice 1, where the marching kernel runs this level),
     // else by its own kernel into v

@@ -106,6 +106,35 @@ def test_box_precond(ctx, boxes, prec):
     assert err <= (1e-12 if prec == "f64" else 1e-5)
 
 
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("edges,levels", [
+    ((4, 8, 12), 1),  # one level below the fine one, of edges 2, 4 and 6
+    ((4, 8, 12), 2),  # the last of edge 1
+    ((16, 24, 8, 20), 2),  # two points per thread, top edges 12 to 4
+    ((16, 32, 8), 3),  # eight points per thread, top edge 16
+    ((40, 24), 2),  # the largest top edge, 20: in FP64 just inside the LDS
+    ((40, 24), 3),  # in FP64 just beyond it
+    ((44,), 1),  # above it in both: level by level
+])
+def test_box_precond_coarse_levels(ctx, edges, levels, prec):
+    """The coarse levels from LDS and, beyond its size, level by level."""
+    gdim, h = (96, 96, 96), (0.3, 0.31, 0.29)
+    rng = np.random.default_rng(23)
+    edge = np.array(edges * 2)[: max(3, len(edges))]
+    m = 1 << levels
+    origin = rng.integers(0, 96 // m, (len(edge), 3)) * m
+    ob = O.Boxes.make(origin, edge, gdim, h)
+    bs = mgx.BoxSet(ctx, origin, edge, gdim, h, levels + 1)
+    r = rng.standard_normal(ob.size(0))
+    for kind, gam in ((0, 0.0), (1, O.gamma(list(ob.h), 1, 0.0, -1.2))):
+        tr, to = to_dev(r), to_dev(np.zeros_like(r))
+        ctx.call("mgx_box_precond_mg", bs.h, kind, levels, gam, CODE[prec], mgx.ptr(tr), mgx.ptr(to))
+        ref = O.b_precond(ob, kind, levels, gam, r, dtype=DT[prec])
+        # the tolerances of test_box_precond: the same cycle, one level deeper at most
+        assert relmax(to_np(to), ref) <= (1e-12 if prec == "f64" else 1e-5), (kind, gam)
+    bs.close()
+
+
 @pytest.mark.parametrize("prec", [mgx.PREC_F64, mgx.PREC_SPLIT])
 def test_box_gram_h_residual(ctx, boxes, cfg, prec):
     ob, bs = boxes

@@ -90,3 +90,30 @@ def test_solver_density(ctx):
     assert np.isfinite(st.band_energy)
     s.close()
     bs.close()
+
+
+@pytest.mark.parametrize("copies, edge, shift", [
+    (1, 20, 2),  # every cell covered, at most 8 boxes: rho is not cleared first
+    (3, 20, 2),  # up to 24 boxes per cell, both loops of the kernel
+    (1, 12, 2),  # cells without a box: their points have to be cleared
+    (1, 20, 1),  # odd origins: single loads
+])
+def test_density_covered_and_uncovered_cells(ctx, copies, edge, shift):
+    """rho holds NaN before the call; tolerance as in this file's head (sums
+    over up to 24 boxes)."""
+    rng = np.random.default_rng(7)
+    g = np.arange(3) * 16
+    base = np.array(np.meshgrid(g, g, g, indexing="ij")).reshape(3, -1).T
+    if edge == 12:
+        base = base[:5]
+    origin = np.concatenate([(base + shift * (i + 1)) % 48 for i in range(copies)])
+    b = O.Boxes.make(origin, np.full(len(origin), edge), (48, 48, 48), 0.3)
+    bs = mgx.BoxSet(ctx, origin, np.full(len(origin), edge), (48, 48, 48), 0.3, 1)
+    psi = rng.standard_normal(b.size(0))
+    a = rng.standard_normal((len(origin),) * 2)
+    rho = to_dev(np.full((48, 48, 48), np.nan))
+    q = bs.density(to_dev(psi), to_dev(np.asfortranarray(a + a.T).ravel(order="F")), rho)
+    ref = O.b_density(b, psi, a + a.T)
+    assert relmax(to_np(rho), ref) <= 1e-13
+    assert q == pytest.approx(O.charge(ref, 0.3**3), rel=1e-11, abs=1e-11 * np.abs(ref).sum() * 0.3**3)
+    bs.close()

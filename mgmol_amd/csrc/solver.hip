@@ -214,7 +214,7 @@ int project(mgx_solver* s, int spec, bool bf16, int& tk)
 }
 
 // The launches of a step up to the host read of its scalars: H psi (with the
-// pending normalisation), S and H, S^-1 (Cholesky + inverse, or spec
+// pending normalisation), S and H, S^-1 (symmetric sweeps, or spec
 // Newton-Schulz steps whose deltas the host checks), theta, the energy, the
 // residual and its norm.  Changes no host state.
 int head_body(mgx_solver* s, bool pending, bool chol, int spec, bool bf16)
@@ -237,7 +237,7 @@ int head_body(mgx_solver* s, bool pending, bool chol, int spec, bool bf16)
     if ((rc = box_gram_h(ctx, s->bs, s->cfg.gram_prec, s->psi, s->hpsi, s->S, s->H, s->Sv, s->Hv))) return rc;
     prof_end(ctx, tk);
     tk = prof_begin(ctx, MGX_PROF_DENSE);
-    // S^-1: Cholesky + inverse (GramMatrix::updateLS / computeInverse), or
+    // S^-1: symmetric sweeps (GramMatrix::updateLS / computeInverse), or
     // the Newton-Schulz refresh from the previous inverse
     if (chol)
     {
@@ -357,7 +357,7 @@ int tail_body(mgx_solver* s, bool use_cnn, bool restored, bool plain_step, doubl
 
 // The same for the Mehrstellen discretisation (FDtype = Mehrstellen): H psi
 // = -Lap_M psi + B V psi and B psi on the boxes, the Galerkin S, H and
-// B-matrix, S^-1 and B-matrix^-1 by Cholesky + inverse (GramMatrix,
+// B-matrix, S^-1 and B-matrix^-1 by symmetric sweeps (GramMatrix,
 // ProjectedMatricesMehrstellen::computeInvB,
 // src/ProjectedMatricesMehrstellen.cc:38-64), theta = B-matrix^-1 H
 // (updateTheta, .h:57-62), the band energy tr(HB S^-1) = tr(theta)

@@ -318,20 +318,29 @@ __global__ void k_tri(double* L, int n, int zero_upper)
     }
 }
 
-// The inverse of a symmetric positive definite block (order m <= 128, its lower
-// triangle read) by symmetric sweeps in registers: pivot k with d = a_kk turns
-// a_ij into a_ij - a_ik a_jk / d, a_ik into a_ik / d and d into -1/d; m sweeps
-// leave minus the inverse.  528 threads each hold a 4 x 4 tile on or below the
-// diagonal; the pivot column goes through LDS (two buffers, one barrier per
-// sweep).  Bound by the sweeps' chain, about 0.5 us each: 62 us at m = 128,
-// where the library's blocked Cholesky and inverse take about 0.5 ms in 50
-// launches.  *info (a double beside the step's scalars): 1 + the first pivot
-// that is not positive, else 0; first: no block came before.
+// A symmetric positive definite block (order m <= 128, its lower triangle
+// read), pivot by pivot in registers.  With the pivot d = a_kk and its row and
+// column w, a_ij becomes a_ij - w_i w_j / d:
+//   FACTOR false  for every i, j (symmetric sweeps): a_ik turns into w_i / d
+//                 and d into -1 / d; m sweeps leave minus the inverse, and P
+//                 receives the inverse;
+//   FACTOR true   for i > k only, which leaves row k of M, the inverse of the
+//                 unit triangle of A = U D U^T, in the places j < k; P
+//                 receives D^-1/2 M = L^-1, A = L L^T the Cholesky
+//                 factorisation (zeros above the diagonal).
+// 528 threads each hold a 4 x 4 tile on or below the diagonal; the pivot's w
+// goes through LDS (two buffers, one barrier per pivot).  Bound by the pivots'
+// chain, about 0.5 us each: 62 us at m = 128, where the library's blocked
+// Cholesky and inverse take about 0.5 ms in 50 launches.  *info (a double
+// beside the step's scalars): 1 + the first pivot that is not positive, else 0;
+// first: no block came before.
 constexpr int kSpdB = 128;
-__global__ void __launch_bounds__(576) k_spd_sweep(const double* A, int64_t ld, int m, double* P, int ldp, double* info,
+template <bool FACTOR>
+__global__ void __launch_bounds__(576) k_spd_block(const double* A, int64_t ld, int m, double* P, int ldp, double* info,
     int k0, int first)
 {
     __shared__ double v[2][kSpdB];
+    __shared__ double piv[FACTOR ? kSpdB : 1];
     // tile (tr, tc), tc <= tr, of thread t = tr (tr + 1) / 2 + tc
     const int t = threadIdx.x;
     int tr      = (int)((sqrtf(8.f * (float)t + 1.f) - 1.f) * 0.5f);
@@ -364,7 +373,7 @@ __global__ void __launch_bounds__(576) k_spd_sweep(const double* A, int64_t ld, 
                 if (tc == k4)
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-                        w[4 * tr + i] = a[i][kk];
+                        w[4 * tr + i] = FACTOR && tr == k4 && i < kk ? a[kk][i] : a[i][kk];
                 else if (tr == k4)
 #pragma unroll
                     for (int j = 0; j < 4; j++)
@@ -373,12 +382,13 @@ __global__ void __launch_bounds__(576) k_spd_sweep(const double* A, int64_t ld, 
             __syncthreads();
             const double d = w[k];
             if (!(d > 0.) && bad == 0. && k < m) bad = (double)(k0 + k + 1);
+            if (FACTOR && t == 0) piv[k] = d;
             // 1 / d: the hardware's estimate and two Newton steps, a third of
             // the division's chain
             double inv = __builtin_amdgcn_rcp(d);
             inv        = __builtin_fma(inv, __builtin_fma(-d, inv, 1.), inv);
             inv        = __builtin_fma(inv, __builtin_fma(-d, inv, 1.), inv);
-            if (!act) continue;
+            if (!act || (FACTOR && tr < k4)) continue;
             double wr[4], wc[4];
 #pragma unroll
             for (int i = 0; i < 4; i++)
@@ -390,8 +400,16 @@ __global__ void __launch_bounds__(576) k_spd_sweep(const double* A, int64_t ld, 
             for (int i = 0; i < 4; i++)
 #pragma unroll
                 for (int j = 0; j < 4; j++)
-                    a[i][j] = __builtin_fma(-wr[i], wc[j], a[i][j]);
+                    if (!FACTOR || tr > k4 || i > kk) a[i][j] = __builtin_fma(-wr[i], wc[j], a[i][j]);
             // the pivot's row and column, in the tiles that hold them
+            if (FACTOR)
+            {
+                if (tc == k4)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (tr > k4 || i > kk) a[i][kk] = -wr[i];
+                continue;
+            }
             if (tc == k4)
 #pragma unroll
                 for (int i = 0; i < 4; i++)
@@ -403,42 +421,45 @@ __global__ void __launch_bounds__(576) k_spd_sweep(const double* A, int64_t ld, 
             if (tr == k4 && tc == k4) a[kk][kk] = -inv;
         }
     }
+    if (FACTOR) __syncthreads();
     if (act)
 #pragma unroll
         for (int i = 0; i < 4; i++)
+        {
+            const int r    = 4 * tr + i;
+            const double s = FACTOR ? 1. / sqrt(piv[r]) : -1.;
 #pragma unroll
             for (int j = 0; j < 4; j++)
             {
-                const int r = 4 * tr + i, c = 4 * tc + j;
-                if (r < m && c <= r)
-                {
-                    P[(int64_t)c * ldp + r] = -a[i][j];
-                    P[(int64_t)r * ldp + c] = -a[i][j];
-                }
+                const int c = 4 * tc + j;
+                if (r >= m || c > r) continue;
+                P[(int64_t)c * ldp + r] = FACTOR && r == c ? s : s * a[i][j];
+                if (!FACTOR || r != c) P[(int64_t)r * ldp + c] = FACTOR ? 0. : s * a[i][j];
             }
+        }
     if (t == 0 && (first || (*info == 0. && bad != 0.))) *info = bad;
 }
 
-// the block column [k0, k0 + m) of X to Q (n x m), its own rows zero
+// the block column [k0, k0 + m) of X to Q (n x m), its own rows the identity
 __global__ void k_spd_panel(const double* X, int n, int k0, int m, double* Q)
 {
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < (int64_t)n * m; t += (int64_t)gridDim.x * blockDim.x)
     {
-        const int row = (int)(t % n);
-        Q[t]          = row >= k0 && row < k0 + m ? 0. : X[(int64_t)k0 * n + t];
+        const int j = (int)(t / n), row = (int)(t - (int64_t)j * n);
+        Q[t]        = row >= k0 && row < k0 + m ? (row - k0 == j ? 1. : 0.) : X[(int64_t)k0 * n + t];
     }
 }
 
-// and back: block column and row from B = Q P, the block from -P
-__global__ void k_spd_panel_back(double* X, int n, int k0, int m, const double* B, const double* P)
+// and back: block column and row from B = Q L^-T L^-1, the block from minus its
+// own rows there
+__global__ void k_spd_panel_back(double* X, int n, int k0, int m, const double* B)
 {
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < (int64_t)n * m; t += (int64_t)gridDim.x * blockDim.x)
     {
         const int j = (int)(t / n), row = (int)(t - (int64_t)j * n);
         const bool in = row >= k0 && row < k0 + m;
-        const double b = in ? -P[(int64_t)j * m + row - k0] : B[t];
-        X[(int64_t)(k0 + j) * n + row] = b;
-        if (!in) X[(int64_t)row * n + k0 + j] = b;
+        X[(int64_t)(k0 + j) * n + row] = in ? -B[t] : B[t];
+        if (!in) X[(int64_t)row * n + k0 + j] = B[t];
     }
 }
 
@@ -1116,23 +1137,28 @@ int chol_inv(mgx_ctx* ctx, int n, const double* S, double* L, double* Sinv)
 }
 
 // X = S^-1 for a symmetric positive definite S (lower triangle read; X apart
-// from S), without its Cholesky factor: one launch up to order 128, else the
-// same sweeps by blocks of 128 (the block's inverse P, the panel B = Q P, the
-// rank-128 update X - B Q^T as a library product, five launches a block).
+// from S), without its Cholesky factor: one launch of symmetric sweeps up to
+// order 128, else in place by blocks of 128.  With A the block as the blocks
+// before it left it, A = L L^T and Q the block's column of X (identity in its
+// own rows): W = Q L^-T, X - W W^T, and the column itself becomes W L^-1.  The
+// part not yet reached is so reduced as by a Cholesky factorisation; with the
+// block's inverse instead (X - Q A^-1 Q^T) it took errors of the order of
+// cond(A) and |I - S X| was 25 times (cond 1e6) to 3e4 times (1e13) the
+// library's at n = 400.  Six launches a block.
 // info (device) receives 1 + the index of the first pivot that is not
-// positive, else 0.  n = 2048: 1.9 ms against the library's 7.3 ms;
-// 512: 0.38 ms against 1.6 ms.
+// positive, else 0.  n = 2048: 2.05 ms against the library's 7.3 ms;
+// 512: 0.42 ms against 1.6 ms.
 int spd_inv_launch(mgx_ctx* ctx, int n, const double* S, double* X, double* info)
 {
     if (n <= kSpdB)
     {
-        hipLaunchKernelGGL(k_spd_sweep, dim3(1), dim3(576), 0, ctx->stream, S, (int64_t)n, n, X, n, info, 0, 1);
+        hipLaunchKernelGGL(k_spd_block<false>, dim3(1), dim3(576), 0, ctx->stream, S, (int64_t)n, n, X, n, info, 0, 1);
         MGX_CHECK_LAUNCH(ctx);
         return MGX_OK;
     }
     double* Q = (double*)workspace(ctx, 7, (2 * (size_t)n * kSpdB + (size_t)kSpdB * kSpdB) * sizeof(double));
     if (!Q) return set_err(ctx, MGX_ENOMEM, "workspace allocation failed");
-    double *B = Q + (size_t)n * kSpdB, *P = B + (size_t)n * kSpdB;
+    double *W = Q + (size_t)n * kSpdB, *Li = W + (size_t)n * kSpdB;
     const double one = 1., zero = 0., mone = -1.;
     rocblas_set_pointer_mode(ctx->blas, rocblas_pointer_mode_host);
     MGX_CHECK_HIP(ctx, hipMemcpyAsync(X, S, (size_t)n * n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
@@ -1140,19 +1166,25 @@ int spd_inv_launch(mgx_ctx* ctx, int n, const double* S, double* X, double* info
     for (int k0 = 0; k0 < n; k0 += kSpdB)
     {
         const int m = std::min(kSpdB, n - k0);
-        hipLaunchKernelGGL(k_spd_sweep, dim3(1), dim3(576), 0, ctx->stream, (const double*)X + (size_t)k0 * n + k0,
-            (int64_t)n, m, P, m, info, k0, k0 == 0);
+        hipLaunchKernelGGL(k_spd_block<true>, dim3(1), dim3(576), 0, ctx->stream, (const double*)X + (size_t)k0 * n + k0,
+            (int64_t)n, m, Li, m, info, k0, k0 == 0);
         hipLaunchKernelGGL(k_spd_panel, dim3(nblocks((int64_t)n * m)), dim3(kBlock), 0, ctx->stream, (const double*)X, n,
             k0, m, Q);
         MGX_CHECK_LAUNCH(ctx);
-        if (rocblas_dgemm(ctx->blas, rocblas_operation_none, rocblas_operation_none, n, m, m, &one, Q, n, P, m, &zero, B, n)
+        // W = Q L^-T, X -= W W^T (the block's own row and column too, which
+        // are written next), Q = W L^-1
+        if (rocblas_dgemm(ctx->blas, rocblas_operation_none, rocblas_operation_transpose, n, m, m, &one, Q, n, Li, m,
+                &zero, W, n)
                 != rocblas_status_success
-            || rocblas_dgemm(ctx->blas, rocblas_operation_none, rocblas_operation_transpose, n, n, m, &mone, B, n, Q, n,
+            || rocblas_dgemm(ctx->blas, rocblas_operation_none, rocblas_operation_transpose, n, n, m, &mone, W, n, W, n,
                    &one, X, n)
+                   != rocblas_status_success
+            || rocblas_dgemm(ctx->blas, rocblas_operation_none, rocblas_operation_none, n, m, m, &one, W, n, Li, m, &zero,
+                   Q, n)
                    != rocblas_status_success)
             return set_err(ctx, MGX_EHIP, "rocblas_dgemm failed");
         hipLaunchKernelGGL(k_spd_panel_back, dim3(nblocks((int64_t)n * m)), dim3(kBlock), 0, ctx->stream, X, n, k0, m,
-            (const double*)B, (const double*)P);
+            (const double*)Q);
     }
     hipLaunchKernelGGL(k_spd_neg, dim3(nblocks((int64_t)n * n)), dim3(kBlock), 0, ctx->stream, X, n);
     MGX_CHECK_LAUNCH(ctx);

@@ -233,8 +233,9 @@ def test_synth_separable_against_oracle_operator(ctx):
 def test_spd_inverse_orders(ctx, n):
     """The inverse without its factor (through mgx_mehr_projected): tiles of 4
     with remainders, one block and several, a last block of one and of a few,
-    only the lower triangle read, in place and apart.  Backward stable sweeps:
-    n * cond * 2^-53 of the largest entry, cond(B) < 20 here, with 4 to spare."""
+    only the lower triangle read, in place and apart.  Errors of a well
+    conditioned inverse, cond(B) < 20 here: n * cond * 2^-53 of the largest
+    entry, with 4 to spare; ill conditioned ones are the next test's."""
     rng = np.random.default_rng(n)
     A = rng.standard_normal((n, 2 * n + 4))
     B = A @ A.T / (2 * n + 4) + 0.2 * np.eye(n)
@@ -255,6 +256,30 @@ def test_spd_inverse_orders(ctx, n):
     ctx.call("mgx_mehr_projected", n, mgx.ptr(tS), mgx.ptr(tI), mgx.ptr(tB), mgx.ptr(tH), mgx.ptr(tB), mgx.ptr(th),
              mgx.ptr(hb), None)
     assert np.array_equal(to_np(tB), got)
+
+
+@pytest.mark.parametrize("cond", [1e6, 1e9])
+@pytest.mark.parametrize("n", [100, 128, 129, 200, 300])
+def test_spd_inverse_ill_conditioned(ctx, n, cond):
+    """|I - B X| against that of the Cholesky inverse (mgx_chol_inv) of the
+    same matrix.  Both are of the order of cond * 2^-53; a constant of 16
+    between them leaves room for the order of the operations (1 to 3 in a CPU
+    restatement), where reducing by a block's explicit inverse loses another
+    cond(block): factors of 60 to 1e6 at these orders beyond 128."""
+    rng = np.random.default_rng(n)
+    q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    B = (q * np.logspace(0, -np.log10(cond), n)) @ q.T
+    B = 0.5 * (B + B.T)
+    tB, t1 = to_dev(B), to_dev(np.eye(n))
+    tL, tX, inv, th, hb = [to_dev(np.zeros((n, n))) for _ in range(5)]
+    ctx.call("mgx_chol_inv", n, mgx.ptr(tB), mgx.ptr(tL), mgx.ptr(tX))
+    ctx.call("mgx_mehr_projected", n, mgx.ptr(t1), mgx.ptr(t1), mgx.ptr(tB), mgx.ptr(t1), mgx.ptr(inv), mgx.ptr(th),
+             mgx.ptr(hb), None)
+    # the products of B and X cancel to 1e-16 cond: formed in extended precision
+    res = [float(np.max(np.abs(np.eye(n) - B.astype(np.longdouble) @ to_np(x).astype(np.longdouble))))
+           for x in (tX, inv)]
+    say("spd", n, cond, res)
+    assert res[1] <= 16 * res[0]
 
 
 @pytest.mark.parametrize("n,k", [(1, 0), (30, 29), (128, 64), (200, 3), (200, 190)])

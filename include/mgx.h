@@ -516,7 +516,10 @@ typedef struct
 int mgx_solver_create(mgx_ctx* ctx, const mgx_boxset* bs, const mgx_solver_cfg_t* cfg,
     const double* vtot_host, const double* psi0_host, mgx_solver** s);
 int mgx_solver_destroy(mgx_solver* s);
-/* one wave-function step; returns residual / energy of the step's input psi */
+/* one wave-function step; returns residual / energy of the step's input psi.
+ * After MGX_ENOTSPD (step and run) the orbitals are the failed step's input,
+ * normalised; the other buffers (H psi, S, H, S^-1, the residual) hold what
+ * the step had computed, and a later step forms S^-1 anew. */
 int mgx_solver_step(mgx_solver* s, mgx_solver_stats_t* st);
 int mgx_solver_run(mgx_solver* s, double tol, int maxit, mgx_solver_stats_t* st);
 /* restart from the initial orbitals (kept on the device) */

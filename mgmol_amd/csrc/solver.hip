@@ -483,9 +483,12 @@ int step_body(mgx_solver* s, double tol, mgx_solver_stats_t* st, bool* done)
     }
     if (rc) return rc;
     MGX_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (chol && (rc = spd_check(ctx, s->host[6]))) return rc;
-    if (mehr && (rc = spd_check(ctx, s->host[7]))) return rc;
-    s->pending_norm = false;
+    s->pending_norm = false;  // psi is normalised (and d the residual's) also where the step fails here
+    if ((chol && (rc = spd_check(ctx, s->host[6]))) || (mehr && (rc = spd_check(ctx, s->host[7]))))
+    {
+        s->have_inv = false;
+        return rc;
+    }
     if (chol)
     {
         s->chol_calls++;
@@ -513,12 +516,16 @@ int step_body(mgx_solver* s, double tol, mgx_solver_stats_t* st, bool* done)
             int steps = 0;
             if (more < 0)
             {
-                if ((rc = spd_inv(ctx, n, s->S, s->Sinv))) return rc;
+                rc    = spd_inv(ctx, n, s->S, s->Sinv);
                 steps = -1;
             }
-            else if ((rc = inverse_update_pairs(ctx, n, s->S, s->Sv, s->tiles, s->Sinv, s->nswork, &steps,
-                          ns_tol, bf16)))
+            else
+                rc = inverse_update_pairs(ctx, n, s->S, s->Sv, s->tiles, s->Sinv, s->nswork, &steps, ns_tol, bf16);
+            if (rc)
+            {
+                s->have_inv = false;
                 return rc;
+            }
             s->ns_steps += spec + std::max(steps, 0);
             if (steps < 0) s->chol_calls++;
             if (more < 0 || steps < 0)
@@ -978,9 +985,10 @@ int mgx_solver_density(mgx_solver* s, double nel, double* rho, double* charge)
     // S of the current psi (FP64; H is a by-product here), its inverse, and
     // dm = 2 S^-1 in theta's buffer
     if ((rc = box_gram_h(ctx, s->bs, MGX_PREC_F64, s->psi, s->psi, s->S, s->H, s->Sv, s->Hv))) return rc;
-    if ((rc = spd_inv(ctx, s->n, s->S, s->Sinv))) return rc;
-    s->have_inv      = true;
-    s->have_xprev    = false;
+    rc            = spd_inv(ctx, s->n, s->S, s->Sinv);
+    s->have_inv   = rc == MGX_OK;
+    s->have_xprev = false;
+    if (rc) return rc;
     const int64_t nn = (int64_t)s->n * s->n;
     hipLaunchKernelGGL(k_scaled_copy, dim3(nblocks(nn)), dim3(kBlock), 0, ctx->stream, (const double*)s->Sinv, nn, 2.,
         s->th);

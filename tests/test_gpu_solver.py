@@ -1,5 +1,7 @@
 """GPU orbital iteration vs the oracle's composed step (FP64 plain mode),
 and convergence of the mixed modes on a small box problem."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -250,3 +252,35 @@ def test_solver_refresh_branches(ctx):
         for s in (chol, capped, free):
             s.close()
         bs.close()
+
+
+@pytest.mark.parametrize("mode", ["chol", "mehr"])
+def test_solver_not_spd_keeps_orbitals(ctx, mode):
+    """A step whose S is singular, with the normalisation of the step before
+    still pending: the call fails with MGX_ENOTSPD and the orbitals are that
+    step's input, normalised once.  All boxes lie on each other and V has one
+    huge value, so the first step's corrections, and with them the next
+    orbitals, agree to rounding."""
+    n, edge, gd, h = 12, 16, 48, 0.3
+    rng = np.random.default_rng(4)
+    psi = rng.uniform(0.5, 1.5, (n, edge, edge, edge))
+    psi /= np.sqrt(h**3 * np.sum(psi * psi, axis=(1, 2, 3)))[:, None, None, None]
+    v = np.zeros((gd,) * 3)
+    v[20, 20, 20] = 1e14
+    origin = np.full((n, 3), 12)
+    bs = mgx.BoxSet(ctx, origin, np.full(n, edge), (gd,) * 3, h, 3)
+    kw = dict(inverse_mode=mgx.INV_CHOL) if mode == "chol" else dict(lap_type=mgx.LAP_MEHRSTELLEN)
+    out = []
+    for steps in (1, 2):
+        s = mgx.Solver(ctx, bs, v, psi, mg_levels=2, precond_dtype=mgx.F64, **kw)
+        if steps == 1:
+            s.run(0.0, 1)
+        else:
+            st = mgx.SolverStats()
+            assert mgx.lib().mgx_solver_run(s.h, 0.0, 2, C.byref(st)) == mgx.MGX_ENOTSPD
+        out.append(s.psi())
+        s.close()
+    norms = h**3 * np.sum(out[1].reshape(n, -1) ** 2, axis=1)
+    assert np.max(np.abs(norms - 1.0)) <= 1e-12
+    assert np.max(np.abs(out[1] - out[0])) <= 1e-13 * np.max(np.abs(out[0]))
+    bs.close()

@@ -667,13 +667,17 @@ int step_body(mgx_solver* s, double tol, mgx_solver_stats_t* st, bool* done)
     return MGX_OK;
 }
 
-// apply a pending normalisation, so that psi is normalised when seen from outside
+// apply a pending normalisation, so that psi is normalised when seen from
+// outside, and wait for the stream: a step ends without a wait of its own (an
+// Anderson update has normalised psi, and then nothing is pending)
 int flush_norm(mgx_solver* s)
 {
-    if (!s->pending_norm) return MGX_OK;
-    int rc = box_scale(s->ctx, s->bs, s->psi, s->d);
-    if (rc) return rc;
-    s->pending_norm = false;
+    if (s->pending_norm)
+    {
+        int rc = box_scale(s->ctx, s->bs, s->psi, s->d);
+        if (rc) return rc;
+        s->pending_norm = false;
+    }
     MGX_CHECK_HIP(s->ctx, hipStreamSynchronize(s->ctx->stream));
     return MGX_OK;
 }
@@ -912,7 +916,10 @@ int mgx_solver_get_psi(mgx_solver* s, double* host)
     if (!s || !host) return MGX_EINVAL;
     int rc = flush_norm(s);
     if (rc) return rc;
-    MGX_CHECK_HIP(s->ctx, hipMemcpy(host, s->psi, s->npts * sizeof(double), hipMemcpyDeviceToHost));
+    // on the engine's stream: it does not wait for the null stream, nor that for it
+    MGX_CHECK_HIP(s->ctx, hipMemcpyAsync(host, s->psi, s->npts * sizeof(double), hipMemcpyDeviceToHost,
+                              s->ctx->stream));
+    MGX_CHECK_HIP(s->ctx, hipStreamSynchronize(s->ctx->stream));
     return MGX_OK;
 }
 

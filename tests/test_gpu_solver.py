@@ -284,3 +284,29 @@ def test_solver_not_spd_keeps_orbitals(ctx, mode):
     assert np.max(np.abs(norms - 1.0)) <= 1e-12
     assert np.max(np.abs(out[1] - out[0])) <= 1e-13 * np.max(np.abs(out[0]))
     bs.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_solver_run_returns_after_the_work(ctx, graph):
+    """Every call returns after its work (the header's promise), also a run
+    that ends on an Anderson step, which leaves no normalisation pending: the
+    stream is idle, and the orbitals read back are the device's."""
+    cfg = synth.box_config(nbox=64, gdim=96, h=0.3, edges=(32,), nwells=8, seed=9, levels=3)
+    bs = mgx.BoxSet(ctx, cfg.origin, cfg.edge, cfg.gdim, cfg.h, 3)
+    s = mgx.Solver(ctx, bs, cfg.vtot, cfg.psi, mg_levels=2, precond_dtype=mgx.F32, anderson_m=1)
+    s.set_graph(graph)
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipStreamQuery.argtypes = [C.c_void_p]
+    stream = C.c_void_p(mgx.lib().mgx_ctx_stream(ctx.h))
+    assert s.run(0.0, 40).dots_sweeps > 0  # Anderson has engaged
+    for k in range(5):
+        s.run(0.0, 2)
+        assert hip.hipStreamQuery(stream) == 0  # hipSuccess, not hipErrorNotReady
+        p = C.c_void_p()
+        host = s.psi()
+        s.ctx.check(mgx.lib().mgx_solver_buffers(s.h, C.byref(p), None, None, None, None, None), "buffers")
+        dev = np.empty_like(host)
+        s.ctx.check(mgx.lib().mgx_memcpy_dtoh(ctx.h, dev.ctypes.data_as(C.c_void_p), p, dev.nbytes), "dtoh")
+        assert np.array_equal(host, dev)
+    s.close()
+    bs.close()

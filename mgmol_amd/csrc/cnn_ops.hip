@@ -1210,8 +1210,8 @@ int mgx_cnn_set_params(mgx_cnn* c, const float* host)
 int mgx_cnn_get_params(mgx_cnn* c, float* host)
 {
     if (!c || !host) return MGX_EINVAL;
-    MGX_CHECK_HIP(c->ctx, hipMemcpy(host, c->p, kNP * sizeof(float), hipMemcpyDeviceToHost));
-    return MGX_OK;
+    MGX_CHECK_HIP(c->ctx, hipMemcpyAsync(host, c->p, kNP * sizeof(float), hipMemcpyDeviceToHost, c->ctx->stream));
+    return sync(c->ctx);
 }
 
 int mgx_cnn_forward(mgx_cnn* c, const float* x, int nb, float* y)
@@ -1251,7 +1251,7 @@ int mgx_cnn_train_step(mgx_cnn* c, const float* x, const float* t, int nb, float
         c->v, kNP, lr, b1, b2, 1e-8f, c1, c2);
     MGX_CHECK_LAUNCH(c->ctx);
     c->dirty = true;
-    return MGX_OK;
+    return sync(c->ctx);
 }
 
 // out_j = rms_j * net(R_j / rms_j) for nbox boxes of edge e packed one after

@@ -161,3 +161,24 @@ def test_cnn_apply_scales_per_box(ctx):
         ref = rms * OC.forward(p, (R[j] / rms)[None].astype(np.float32), bf16_mode=True)[0][0]
         assert _rel(out[j], ref) < 5e-3, j
     net.close()
+
+
+def test_cnn_train_step_returns_after_the_work(ctx):
+    """The stream is idle after a training step (the parameters' update is its
+    last launch), and the parameters read back are the updated ones."""
+    import ctypes as C
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((2, 12, 12, 12)).astype(np.float32)
+    p = _params(3)
+    net = learned.Cnn(ctx, 12, 2, p)
+    tx, tt = to_dev(x), to_dev(0.5 * x)
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipStreamQuery.argtypes = [C.c_void_p]
+    last = p
+    for _ in range(5):
+        net.train_step(tx.data_ptr(), tt.data_ptr(), 2, 1e-3)
+        assert hip.hipStreamQuery(C.c_void_p(mgx.lib().mgx_ctx_stream(ctx.h))) == 0
+        now = net.params()
+        assert all(not np.array_equal(now[k], last[k]) for k in learned.NAMES)
+        last = now
+    net.close()

@@ -12,6 +12,7 @@
 #include "common.hpp"
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <type_traits>
 
@@ -75,6 +76,15 @@ struct mgx_boxset
     int* d_sp_col    = nullptr;
     int* d_sp_k      = nullptr;
     int* d_sp_e      = nullptr;
+    // behind the tiles in d_sp_col, from cls_at on, per level: the boxes in the
+    // same order grouped by the size class of their edge at that level
+    // (k_box_coarse); per class its first place, count and largest edge
+    struct CoarseClass
+    {
+        int first = 0, n = 0, edge = 0;
+    };
+    std::vector<std::array<CoarseClass, 3>> cls;
+    size_t cls_at    = 0;
     // autotuned launch shapes (MGX_TUNE_*) and whether the tuner ran or a
     // caller set them
     int tune[MGX_TUNE_N] = { 1, 1, 1, 1, 1, 1, 1, 1 };
@@ -91,6 +101,14 @@ namespace
 
 constexpr double kInv12 = 1. / 12.;
 constexpr double kInv64 = 1. / 64.;
+
+// size classes of a box's edge at the top of its coarse levels, and the points
+// per thread there: short columns while the block is not full (edge 12, 128
+// boxes: 8.3 us with 2, 9 with 4, 33 with 8 points at once); a block of 1024 at
+// most beyond (edge 16, 2048 boxes, FP32: 78 us with 4 points, 57 with 8).
+// Larger boxes (third class up to kCoarseEdge) are swept level by level.
+constexpr int kCoarseEdge = 20, kCoarseK[3] = { 2, 8, 10 };
+int coarse_class(int e) { return e <= 12 ? 0 : e <= 16 ? 1 : 2; }
 
 int wrap_h(int i, int n)
 {
@@ -1107,13 +1125,12 @@ __global__ void k_first_sweep(const double* res, T* f, T* x, int64_t n, double j
 //
 // Measured, all coarse levels of one cycle: 2048 boxes of edge 32 (top edge
 // 16, FP32) 115 us in 11 launches, 57 in this one (92 with f and every
-// neighbour from LDS); 512 boxes of 24 to 40 (FP64) 132 -> 92; 128 of 20 and
+// neighbour from LDS); 512 boxes of 24 to 40 (FP64) 132 -> 91; 128 of 20 and
 // 24 (FP64) 70 -> 8; 24 of 8 to 16 (FP32) 40 -> 5.  Left at the top: FP64
 // adds and multiplies and the LDS reads of y and z; one block of 1024 threads
 // per CU at top edge 20, whose FP64 columns spill (f and x from LDS instead:
 // 148 us).
 constexpr int kCoarseLevels = 8;
-constexpr int kCoarseLds    = 160 * 1024;
 
 struct CoarseArgs
 {
@@ -1293,9 +1310,10 @@ struct CoarseCol
     }
 };
 
-// K points per thread on the top level
+// K points per thread on the top level; the second size class (K = 8) has blocks
+// of 512 and so the registers for its FP64 columns
 template <typename T, int K>
-__global__ void __launch_bounds__(1024) k_box_coarse(const T* __restrict__ f, T* __restrict__ out, CoarseArgs a)
+__global__ void __launch_bounds__(K == 8 ? 512 : 1024) k_box_coarse(const T* __restrict__ f, T* __restrict__ out, CoarseArgs a)
 {
     static_assert(K % 2 == 0, "a column starts on an even plane");
     extern __shared__ unsigned char lds_raw[];
@@ -3599,9 +3617,20 @@ int box_mg_setup(mgx_ctx* ctx, const mgx_boxset* bs, int max_levels, BoxMG<T>& B
 }
 
 // The levels from `level` on (the coarse ones: 2nd order operator, zero start,
-// the iterate of `level` to out) by k_box_coarse; false where a box's levels
-// do not fit its LDS or a thread's points its registers.  FP32 and FP64 only:
-// the FP16 cycle rounds its FP32 arithmetic at other places.
+// the iterate of `level` to out) by k_box_coarse, in one launch or one per size
+// class; false where a box's edge there is above kCoarseEdge (a thread's points
+// would not fit its registers).  FP32 and FP64 only: the FP16 cycle rounds its
+// FP32 arithmetic at other places.
+//
+// A launch's threads and LDS are those of its largest box, so all boxes go in
+// one launch only while the chip holds their blocks at once: 8 boxes of 40 with
+// 2000 of 8 (top edges 20 and 4, FP64) took 566 us in one launch and 342 in
+// two, level by level 377 (the whole V-cycle); 512 boxes of 24 to 40 (FP64) 694
+// and 665.  Up to there the further launches cost more (128 boxes of 24 to 40:
+// 236 us in one, 252 in three; 256 of 20 and 32: 170 and 175).  Blocks at once:
+// 256, FP32 ones of the second class 512 (512 boxes of 16 with some of 32: 171
+// and 173; 768: 196 and 191), FP64 ones of the third somewhat fewer than 256
+// (192 boxes of 24 to 40: 264 and 285; 224: 311 and 305).
 template <typename T>
 bool box_coarse(mgx_ctx* ctx, const mgx_boxset* bs, int level, int max_levels, const T* f, T* out, int* rc, bool run)
 {
@@ -3610,17 +3639,7 @@ bool box_coarse(mgx_ctx* ctx, const mgx_boxset* bs, int level, int max_levels, c
     {
         CoarseArgs a;
         a.nl = max_levels - level + 1;
-        const int e = bs->maxedge >> level;
-        if (a.nl > kCoarseLevels || e > 20) return false;
-        // short columns while the block is not full (edge 12, 128 boxes: 8.3 us
-        // with 2, 9 with 4, 33 with 8 points at once); a block of 1024 at most
-        // beyond (edge 16, 2048 boxes, FP32: 78 us with 4 points, 57 with 8)
-        const int K = e <= 12 ? 2 : e <= 16 ? 8 : 10;
-        // every term grows with the edge: the largest box's are enough
-        const int elems    = std::max({ coarse_lds(e, a.nl), coarse_span(e, K),
-            a.nl > 1 ? coarse_x_size(e) + coarse_span(e / 2, K / 2) : 0 });
-        const size_t bytes = sizeof(T) * (size_t)elems;
-        if (bytes > (size_t)kCoarseLds) return false;
+        if (a.nl > kCoarseLevels || (bs->maxedge >> level) > kCoarseEdge) return false;
         if (!run) return true;
         for (int l = 0; l < a.nl; l++)
         {
@@ -3629,19 +3648,35 @@ bool box_coarse(mgx_ctx* ctx, const mgx_boxset* bs, int level, int max_levels, c
             a.jf[l]           = jacobi_factor(MGX_LAP_2ND, h);
             a.c2[l]           = coef2(h);
         }
-        a.off = bs->d_off[level], a.edge = bs->d_edge, a.order = bs->d_sp_col;
-        a.shift = level, a.nbox = bs->nbox;
-        const int nt      = std::max(e * e * ((e + K - 1) / K), a.nl > 1 ? (e / 2) * (e / 2) * (e / 2) : 0);
-        const int NT      = (nt + 63) / 64 * 64;
-        const auto kernel = K == 2 ? k_box_coarse<T, 2> : K == 8 ? k_box_coarse<T, 8> : k_box_coarse<T, 10>;
-        if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes)
-            != hipSuccess)
+        a.off = bs->d_off[level], a.edge = bs->d_edge, a.shift = level;
+        *rc   = MGX_OK;
+        const int last   = coarse_class(bs->maxedge >> level);
+        const int at_once = sizeof(T) == 8 ? (last == 2 ? 208 : 256) : (last == 2 ? 256 : 512);
+        const bool split  = bs->nbox > at_once;
+        for (int c = split ? 0 : last; c <= last; c++)
         {
-            *rc = set_err(ctx, MGX_EHIP, "k_box_coarse: LDS size");
-            return true;
+            auto cl = bs->cls[level][c];
+            if (!cl.n) continue;
+            if (!split) cl.first = 0, cl.n = bs->nbox;
+            const int e = cl.edge, K = kCoarseK[c];
+            a.order = bs->d_sp_col + bs->cls_at + (size_t)level * bs->nbox + cl.first, a.nbox = cl.n;
+            // every term grows with the edge: the largest box's are enough
+            // (101 KB at most, at edge 20 in FP64)
+            const int elems    = std::max({ coarse_lds(e, a.nl), coarse_span(e, K),
+                a.nl > 1 ? coarse_x_size(e) + coarse_span(e / 2, K / 2) : 0 });
+            const size_t bytes = sizeof(T) * (size_t)elems;
+            const int nt       = std::max(e * e * ((e + K - 1) / K), a.nl > 1 ? (e / 2) * (e / 2) * (e / 2) : 0);
+            const int NT       = (nt + 63) / 64 * 64;
+            const auto kernel  = c == 0 ? k_box_coarse<T, kCoarseK[0]>
+                                        : c == 1 ? k_box_coarse<T, kCoarseK[1]> : k_box_coarse<T, kCoarseK[2]>;
+            if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes)
+                != hipSuccess)
+            {
+                *rc = set_err(ctx, MGX_EHIP, "k_box_coarse: LDS size");
+                return true;
+            }
+            hipLaunchKernelGGL(kernel, dim3((cl.n + 7) / 8 * 8), dim3(NT), bytes, ctx->stream, f, out, a);
         }
-        hipLaunchKernelGGL(kernel, dim3((bs->nbox + 7) / 8 * 8), dim3(NT), bytes, ctx->stream, f, out, a);
-        *rc = MGX_OK;
         return true;
     }
 }
@@ -4663,6 +4698,27 @@ int mgx_boxset_create(mgx_ctx* ctx, const mgx_boxes_t* b, int levels, mgx_boxset
                 pos[r] = -1;
         }
         tptr[s->ntile] = (int)tk.size();
+        // the same order by size class, a list per level behind the tiles
+        s->cls.resize(levels);
+        s->cls_at = tcol.size();
+        for (int l = 0; l < levels; l++)
+        {
+            int at = 0;
+            for (int c = 0; c < 3; c++)
+            {
+                auto& k = s->cls[l][c];
+                k.first = at;
+                for (auto& kj : key)
+                {
+                    const int e = s->edge[kj.second] >> l;
+                    if (coarse_class(e) != c) continue;
+                    tcol.push_back(kj.second);
+                    at++;
+                    k.edge = std::max(k.edge, e);
+                }
+                k.n = at - k.first;
+            }
+        }
         if (hipMalloc(&s->d_sp_ptr, sizeof(int) * tptr.size()) != hipSuccess
             || hipMalloc(&s->d_sp_col, sizeof(int) * tcol.size()) != hipSuccess
             || hipMalloc(&s->d_sp_k, sizeof(int) * std::max<size_t>(tk.size(), 1)) != hipSuccess

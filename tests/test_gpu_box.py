@@ -135,6 +135,38 @@ def test_box_precond_coarse_levels(ctx, edges, levels, prec):
     bs.close()
 
 
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("edges,levels", [
+    ((40,) + (8,) * 9, 2),  # one large box among small ones, in one launch
+    ((24, 32, 40, 16, 36, 28), 2),  # the three size classes (top edges up to 12, 16, 20), in one launch
+    ((40, 36, 32, 28, 24) + (8,) * 260, 2),  # more boxes than CUs: a launch per class
+    ((40, 28) + (4, 8) * 130, 1),  # the same, the coarse levels one level
+    ((32,) * 2 + (16,) * 260, 3),  # the second class and the first, FP64 in two launches
+    ((32,) * 2 + (8,) * 520, 1),  # and both types
+    ((40, 24) + (8, 12) * 110, 2),  # between the two limits, FP64 by class and FP32 not
+])
+def test_box_precond_size_classes(ctx, edges, levels, prec):
+    """The coarse levels from LDS, in one launch and in one per size class of
+    the top edge: every box in its own class, in any order."""
+    gdim, h = (96, 96, 96), (0.3, 0.31, 0.29)
+    rng = np.random.default_rng(29)
+    edge = rng.permutation(np.array(edges))
+    m = 1 << levels
+    origin = rng.integers(0, 96 // m, (len(edge), 3)) * m
+    ob = O.Boxes.make(origin, edge, gdim, h)
+    bs = mgx.BoxSet(ctx, origin, edge, gdim, h, levels + 1)
+    r = rng.standard_normal(ob.size(0))
+    tr, to = to_dev(r), to_dev(np.full_like(r, np.nan))
+    ctx.call("mgx_box_precond_mg", bs.h, 1, levels, 0.0, CODE[prec], mgx.ptr(tr), mgx.ptr(to))
+    ref = O.b_precond(ob, 1, levels, 0.0, r, dtype=DT[prec])
+    # the tolerances of test_box_precond, per box
+    off = ob.offsets()
+    for j in range(len(edge)):
+        a, b = off[j], off[j + 1]
+        assert relmax(to_np(to)[a:b], ref[a:b]) <= (1e-12 if prec == "f64" else 1e-5), (j, edge[j])
+    bs.close()
+
+
 @pytest.mark.parametrize("prec", [mgx.PREC_F64, mgx.PREC_SPLIT])
 def test_box_gram_h_residual(ctx, boxes, cfg, prec):
     ob, bs = boxes

@@ -1059,9 +1059,19 @@ int tsgemm(mgx_ctx* ctx, int prec, const double* A, const double* B, int64_t ld,
     MGX_REQUIRE(ctx, (int64_t)subdivx * lnp <= ld, "slabs exceed the leading dimension");
     MGX_REQUIRE(ctx, prec == MGX_PREC_F64 || prec == MGX_PREC_SPLIT, "bad precision mode");
     if (n >= kWideN) return tsgemm_wide(ctx, prec, A, B, ld, lnp, n, subdivx, vel, ss);
-    // the fewest panels of at most four tiles, all of one width
-    const int ntile = (n + 15) / 16, npan = (ntile + 3) / 4, tw = (ntile + npan - 1) / npan;
-    const int pairs = lower_only ? npan * (npan + 1) / 2 : npan * npan;
+    // the fewest panels of at most four tiles, all of one width.  With few rows
+    // a wide pair is a chain of up to 16 tiles' MFMAs per 16 rows beside an idle
+    // chip: single tiles where wide pairs would give under 176 (split: 224)
+    // blocks of 256 rows.  Product of 100 columns of 1000 rows, split: 49 us in
+    // wide pairs, 19 in single tiles; near the line, Gram of 200 columns of 6000
+    // rows, split (230 blocks): 53 and 40; product of 48 columns of 50000 rows,
+    // FP64 (195 blocks): 32 and 37.
+    const int ntile = (n + 15) / 16;
+    int npan = (ntile + 3) / 4, tw = (ntile + npan - 1) / npan;
+    auto npairs = [&]() { return lower_only ? npan * (npan + 1) / 2 : npan * npan; };
+    const int64_t wide = npairs() * subdivx * std::max<int64_t>(1, lnp / 256);
+    if (wide < (prec == MGX_PREC_F64 ? 176 : 224)) npan = ntile, tw = 1;
+    const int pairs = npairs();
     // blocks of four waves: as many per CU as the tiles' registers let reside
     // (1, 2, 3, 6 for widths 4..1), each wave at least four chunks of 16 rows
     static const int percu[4] = { 6, 3, 2, 1 };

@@ -54,11 +54,14 @@ def test_local_gram_and_product_f64(ctx, n, ld, lnp, sub):
 @pytest.mark.parametrize("prec", [mgx.PREC_F64, mgx.PREC_SPLIT])
 @pytest.mark.parametrize("n,ld,lnp,sub", [(1, 40, 7, 1), (3, 5000, 4999, 1), (16, 640, 320, 2), (17, 301, 100, 3),
                                           (33, 2048, 2048, 1), (48, 1031, 515, 2), (65, 4100, 4100, 1),
-                                          (97, 777, 777, 1), (130, 600, 299, 2), (255, 1500, 1500, 1)])
+                                          (97, 777, 777, 1), (130, 600, 299, 2), (255, 1500, 1500, 1),
+                                          (100, 20000, 20000, 1), (64, 60000, 60000, 1), (200, 4800, 300, 16),
+                                          (48, 57000, 57000, 1)])
 def test_local_products_panels(ctx, prec, n, ld, lnp, sub):
-    """Every panel width (1 to 4 tiles), one to four panels, ragged last tiles
-    and panels, rows not multiples of 16, odd leading dimensions and slab
-    starts (unaligned columns), fewer rows than one chunk.  FP64: 1e-13 of the
+    """Every panel width (1 to 4 tiles; single tiles with few rows, on both
+    sides of the line), one to four panels, ragged last tiles and panels, rows
+    not multiples of 16, odd leading dimensions and slab starts (unaligned
+    columns), fewer rows than one chunk.  FP64: 1e-13 of the
     largest entry as above; split: 2^-24 relative per product, FP32 sums of 16
     (hi * hi) and 32 (hi * lo) products: 20 * 2^-24 of the sum of |a||b| bounds
     it, here 1.2e-6 of the largest entry of |A|^T |B|."""

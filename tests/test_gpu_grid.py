@@ -282,17 +282,28 @@ def test_precond_packed(ctx, prec, lap, dims, nf, levels, bc):
     assert np.array_equal(to_np(tr)[:, n:], res[:, n:])
 
 
-def test_precond_overlapping_buffers(ctx):
-    """Results over a shifted residual: the general path, as before."""
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("shift,pad", [(64, 0), (-64, 0), (1, 3), (4096 + 5, 10)])
+def test_precond_overlapping_buffers(ctx, prec, shift, pad):
+    """Results over a shifted residual, before and behind it, by one value, and
+    by a whole function: from a copy of the residual (FP64) or the general path
+    (FP32); the tolerances of test_precond_packed."""
     og, mg_ = _grids(dims=(16, 16, 16), ll=4.8)
-    n = og.size
+    n, nf = og.size, 3
+    ld = n + pad
     rng = np.random.default_rng(3)
-    buf = rng.standard_normal(n + 64)
+    buf = rng.standard_normal(nf * ld + abs(shift))
+    r0 = max(0, -shift)
+    res = np.ascontiguousarray(buf[r0:r0 + nf * ld].reshape(nf, ld)[:, :n])
     gam = O.gamma(list(og.h), 2, 0.0, -1.0)
     t = to_dev(buf)
-    ctx.call("mgx_precond_mg", 2, 2, gam, mgx.F64, mg_, mgx.ptr(t), n, 1, None, C.c_void_p(t.data_ptr() + 64 * 8), n)
-    ref = O.precond(og, 2, 2, gam, buf[None, :n], dtype=DT["f64"])
-    assert relmax(to_np(t)[64:], ref[0]) <= 1e-12
+    at = lambda k: C.c_void_p(t.data_ptr() + 8 * k)
+    ctx.call("mgx_precond_mg", 2, 2, gam, mgx.F32 if prec == "f32" else mgx.F64, mg_, at(r0), ld, nf, None,
+             at(r0 + shift), ld)
+    ref = O.precond(og, 2, 2, gam, res, dtype=DT[prec])
+    o = r0 + shift
+    got = np.concatenate([to_np(t), np.zeros(pad)])[o:o + nf * ld].reshape(nf, ld)
+    assert relmax(got[:, :n], ref) <= (1e-12 if prec == "f64" else 1e-5)
 
 
 def test_precond_refuses_what_it_refused(ctx):

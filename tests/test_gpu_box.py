@@ -112,17 +112,21 @@ def test_box_precond(ctx, boxes, prec):
     ((4, 8, 12), 2),  # the last of edge 1
     ((16, 24, 8, 20), 2),  # two points per thread, top edges 12 to 4
     ((16, 32, 8), 3),  # eight points per thread, top edge 16
-    ((40, 24), 2),  # the largest top edge, 20: in FP64 just inside the LDS
-    ((40, 24), 3),  # in FP64 just beyond it
-    ((44,), 1),  # above it in both: level by level
+    ((40, 24), 2),  # the largest top edge that goes from LDS, 20
+    ((40, 24), 3),  # with the most LDS, 98 KB in FP64
+    ((44,), 1),  # a top edge above it: level by level
+    ((48,), 2),  # level 1 (edge 24) by launches, level 2 (edge 12) from LDS
+    ((44, 24), 2),  # the same with small boxes: edges 22 and 12, then 11 and 6
+    ((48, 24), 3),  # levels 2 and 3 from LDS below a level by launches
 ])
 def test_box_precond_coarse_levels(ctx, edges, levels, prec):
-    """The coarse levels from LDS and, beyond its size, level by level."""
-    gdim, h = (96, 96, 96), (0.3, 0.31, 0.29)
+    """The coarse levels from LDS, above the largest top edge level by level,
+    and a level by launches above levels from LDS."""
+    gdim, h = (104, 104, 104), (0.3, 0.31, 0.29)
     rng = np.random.default_rng(23)
     edge = np.array(edges * 2)[: max(3, len(edges))]
     m = 1 << levels
-    origin = rng.integers(0, 96 // m, (len(edge), 3)) * m
+    origin = rng.integers(0, 104 // m, (len(edge), 3)) * m
     ob = O.Boxes.make(origin, edge, gdim, h)
     bs = mgx.BoxSet(ctx, origin, edge, gdim, h, levels + 1)
     r = rng.standard_normal(ob.size(0))

@@ -285,11 +285,41 @@ def test_spd_inverse_ill_conditioned(ctx, n, cond):
     assert res[1] <= 16 * res[0]
 
 
-@pytest.mark.parametrize("n,k", [(1, 0), (30, 29), (128, 64), (200, 3), (200, 190)])
-def test_spd_inverse_rejects_indefinite(ctx, n, k):
-    B = 2.0 * np.eye(n)
-    B[k, k] = -1.0
-    t = [to_dev(x) for x in (B, np.eye(n), B, B)]
+@pytest.mark.parametrize("n,i,j", [
+    (1, 0, 0), (200, 3, 3), (200, 190, 190),  # a negative value on the diagonal
+    (30, 4, 5), (128, 0, 127), (128, 126, 127),  # coupled within the block: the pivot updates decide
+    (200, 1, 127), (200, 130, 199),  # within the first and the last of several blocks
+    (200, 5, 150), (300, 127, 128), (300, 60, 299),  # across blocks: the panels and the updates between decide
+])
+@pytest.mark.parametrize("coupling", [1.0 + 1e-6, 1.0 - 1e-6])
+def test_spd_inverse_rejects_indefinite(ctx, n, i, j, coupling):
+    """Two unit-diagonal rows coupled by a little more and a little less than
+    one, beside a well conditioned coupling of all: indefinite, and just
+    definite, whose inverse has to be as good as its condition allows (4 n *
+    cond * 2^-53 of its largest entry)."""
+    rng = np.random.default_rng(n + i)
+    G = rng.standard_normal((n, 2 * n))
+    B = np.eye(n) + 0.05 * (G @ G.T) / (2 * n)
+    if i == j:
+        B[i, i] = -coupling
+    else:
+        B[[i, j]] = 0.0
+        B[:, [i, j]] = 0.0
+        B[i, i] = B[j, j] = 1.0
+        B[i, j] = B[j, i] = coupling
+        # a congruence: the sign of the pair's determinant shows only after the
+        # other rows' updates
+        T = np.eye(n)
+        T[[i, j]] += 0.1 * rng.standard_normal((2, n)) / np.sqrt(n)
+        B = T.T @ B @ T
+        B = 0.5 * (B + B.T)
+    t = [to_dev(x) for x in (np.eye(n), np.eye(n), B, np.eye(n))]
     o = [to_dev(np.zeros((n, n))) for _ in range(3)]
     rc = mgx.lib().mgx_mehr_projected(ctx.h, n, *[mgx.ptr(x) for x in t + o], None)
-    assert rc == mgx.MGX_ENOTSPD
+    w = np.linalg.eigvalsh(B)
+    assert (w[0] < 0.0) == (coupling > 1.0 or i == j)
+    if w[0] < 0.0:
+        assert rc == mgx.MGX_ENOTSPD
+    else:
+        assert rc == 0
+        assert relmax(to_np(o[0]), np.linalg.inv(B)) <= 4 * n * (w[-1] / w[0]) * 2.0 ** -53

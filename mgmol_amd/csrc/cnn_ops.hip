@@ -30,7 +30,6 @@ namespace mgx
 namespace
 {
 
-constexpr int kCh      = 16;
 constexpr int kTaps    = 27;
 constexpr int kWaves   = 4;  // per block
 constexpr int kDwBlocks = 512;  // most blocks of a 16 -> 16 weight gradient: two per CU
@@ -40,7 +39,6 @@ constexpr int kDwPad    = 256;  // bytes after the activations that its last row
 constexpr int kW0 = 0, kB0 = kW0 + 27 * 16, kW1 = kB0 + 16, kB1 = kW1 + 27 * 256, kW2 = kB1 + 16,
               kB2 = kW2 + 27 * 256, kW3 = kB2 + 16, kB3 = kW3 + 27 * 16, kS = kB3 + 1, kNP = kS + 1;
 
-typedef short s4 __attribute__((ext_vector_type(4)));
 typedef short s8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
@@ -60,14 +58,6 @@ __host__ __device__ inline uint16_t f2bf(float f)
     memcpy(&u, &f, 4);
     u += 0x7FFFu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
-}
-
-__host__ __device__ inline float bf2f(uint16_t h)
-{
-    const uint32_t u = (uint32_t)h << 16;
-    float f;
-    memcpy(&f, &u, 4);
-    return f;
 }
 
 __device__ inline int tap_dx(int t) { return t / 9 - 1; }
@@ -931,13 +921,6 @@ __global__ void k_box_scale_to_f32(const double* R, const double* rms, int64_t m
         x[i] = (float)(R[i] / rms[i / m]);
 }
 
-template <typename T>
-__global__ void k_box_scale_from_f32(const float* y, const double* rms, int64_t m, int64_t n, T* out)
-{
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        out[i] = (T)((double)y[i] * rms[i / m]);
-}
-
 }  // namespace
 }  // namespace mgx
 
@@ -952,7 +935,7 @@ struct mgx_cnn
     uint16_t *f0, *f1, *f2, *f3, *r3, *r2, *r1;
     // activations for max_batch samples
     uint16_t *h1 = nullptr, *h2 = nullptr, *h3 = nullptr, *dza = nullptr, *dzb = nullptr;
-    float *z = nullptr, *y = nullptr, *dy = nullptr, *xf = nullptr;
+    float *z = nullptr, *dy = nullptr;
     float *part0 = nullptr, *part1 = nullptr, *part2 = nullptr, *part3 = nullptr;  // weight-gradient partials per layer
     double *lpart = nullptr, *rms = nullptr;
     double* host  = nullptr;  // pinned
@@ -1149,9 +1132,7 @@ int mgx_cnn_create(mgx_ctx* ctx, int edge, int max_batch, mgx_cnn** out)
     al((void**)&c->dza, nv * 16 * sizeof(uint16_t) + kDwPad);
     al((void**)&c->dzb, nv * 16 * sizeof(uint16_t) + kDwPad);
     al((void**)&c->z, nv * sizeof(float));
-    al((void**)&c->y, nv * sizeof(float));
     al((void**)&c->dy, nv * sizeof(float));
-    al((void**)&c->xf, nv * sizeof(float));
     al((void**)&c->part0, nd1 * sizeof(float));
     al((void**)&c->part1, nd16 * sizeof(float));
     al((void**)&c->part2, nd16 * sizeof(float));
@@ -1186,8 +1167,8 @@ int mgx_cnn_create(mgx_ctx* ctx, int edge, int max_batch, mgx_cnn** out)
 int mgx_cnn_destroy(mgx_cnn* c)
 {
     if (!c) return MGX_OK;
-    void* bufs[] = { c->p, c->g, c->m, c->v, c->wbf, c->h1, c->h2, c->h3, c->dza, c->dzb, c->z, c->y, c->dy, c->xf,
-        c->part0, c->part1, c->part2, c->part3, c->lpart, c->rms };
+    void* bufs[] = { c->p, c->g, c->m, c->v, c->wbf, c->h1, c->h2, c->h3, c->dza, c->dzb, c->z, c->dy, c->part0,
+        c->part1, c->part2, c->part3, c->lpart, c->rms };
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (c->host) (void)hipHostFree(c->host);

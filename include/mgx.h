@@ -30,7 +30,7 @@ extern "C" {
 #define MGX_OK 0
 #define MGX_EINVAL -1   /* bad argument (reference: assert / exit(2)) */
 #define MGX_EHIP -2     /* HIP runtime or library failure */
-#define MGX_ENOTSPD -3  /* Cholesky failed: S not SPD (reference: mmpi.abort) */
+#define MGX_ENOTSPD -3  /* S (or B) not positive definite (reference: mmpi.abort) */
 #define MGX_ENUMERIC -4 /* NaN/Inf detected, or a density charge off the electron count */
 #define MGX_ENOMEM -5   /* device allocation failed */
 
@@ -271,7 +271,7 @@ int mgx_mehr_bmatrix(mgx_ctx* ctx, const mgx_grid_t* grid, const double* psi, in
     double* B);
 /* ProjectedMatricesMehrstellen::computeInvB / updateTheta / updateHB,
  * src/ProjectedMatricesMehrstellen.cc:38-64, .h:46-69, and getEigSum,
- * src/ProjectedMatrices.cc:550-569: invB = B^-1 (Cholesky; MGX_ENOTSPD),
+ * src/ProjectedMatrices.cc:550-569: invB = B^-1 (MGX_ENOTSPD),
  * theta = invB H, HB = (S theta + (S theta)^T) / 2, *eigsum (host, may be
  * NULL) = tr(HB Sinv) [Ry] */
 int mgx_mehr_projected(mgx_ctx* ctx, int n, const double* S, const double* Sinv, const double* B,
@@ -438,8 +438,9 @@ typedef struct
     int precond_kind;    /* MGX_PRECOND_VCYCLE, or MGX_PRECOND_LEARNED (mgx_solver_set_cnn) */
     int inverse_mode;    /* S^-1 after the first step: MGX_INV_NS_F64 (Newton-Schulz refresh,
                             FP64 products), MGX_INV_NS_BF16 (its correction as one BF16 hi/lo
-                            product, no counterpart in the reference) or MGX_INV_CHOL (Cholesky +
-                            inverse every step, GramMatrix::updateLS / computeInverse) */
+                            product, no counterpart in the reference) or MGX_INV_CHOL (from
+                            S itself every step, what GramMatrix::updateLS / computeInverse
+                            leave, without the factor) */
     double ns_tol;       /* Newton-Schulz target max|I - S^-1 S|; 0 = 1e-15 with FP64 S,
                             1e-10 with the split S */
     int ns_max_spec;     /* most refresh steps taken before the host checks them (0 = 4) */
@@ -478,7 +479,7 @@ typedef struct
  * or flops for LEARNED, NSGEMM and NSGEMM16 (mgx_solver_profile_work). */
 #define MGX_PROF_HLOC 0      /* H psi (one marching kernel) */
 #define MGX_PROF_GRAM 1      /* S, H pair contractions */
-#define MGX_PROF_DENSE 2     /* Cholesky, inverse, theta, trace, Ritz */
+#define MGX_PROF_DENSE 2     /* inverse, theta, trace, Ritz */
 #define MGX_PROF_RESID 3     /* residual + norm */
 #define MGX_PROF_JACOBI0 4   /* fine-level Jacobi sweeps without the Anderson dots */
 #define MGX_PROF_PRECOND 5   /* whole V-cycle incl. update */
@@ -507,10 +508,10 @@ typedef struct
     int learned_steps;   /* CNN trials (accepted or not), cumulative */
     int fallbacks;       /* CNN trials whose step lost to the V-cycle step from the same state */
     int ns_steps;        /* Newton-Schulz refresh steps of S^-1 (one dgemm each), cumulative */
-    int chol_calls;      /* Cholesky + inverse of S (first step and refresh failures), cumulative */
+    int chol_calls;      /* inverses formed from S itself (first step and refresh failures), cumulative */
     int dots_sweeps;     /* V-cycles whose last fine sweep also formed the Anderson dots, cumulative */
     int ns_continued;    /* refreshes whose unchecked steps fell short and were continued with checks */
-    int ns_restarts;     /* refreshes that diverged and were replaced by Cholesky + inverse */
+    int ns_restarts;     /* refreshes that diverged and were replaced by an inverse from S itself */
 } mgx_solver_stats_t;
 
 int mgx_solver_create(mgx_ctx* ctx, const mgx_boxset* bs, const mgx_solver_cfg_t* cfg,
@@ -546,19 +547,20 @@ int mgx_solver_buffers(mgx_solver* s, double** psi, double** hpsi, double** S, d
  * per step, the same values.  No counterpart in the reference. */
 int mgx_solver_set_keep_residual(mgx_solver* s, int on);
 /* device pointer of the solver's S^-1 (n x n, column-major): the inverse of the
- * S of the last evaluated step (refreshed, or Cholesky) */
+ * S of the last evaluated step (refreshed, or from S itself) */
 int mgx_solver_inverse(mgx_solver* s, double** Sinv);
 /* replace the orbitals (host, the box set's packed layout), e.g. extrapolated
  * orbitals after an ionic move (MGmol::extrapolate_orbitals keeps the solver
  * state); the Anderson history is cleared, S^-1 stays as the start of the next
- * refresh (which falls back to Cholesky when it is too far off) */
+ * refresh (which falls back to S itself when it is too far off) */
 int mgx_solver_set_psi(mgx_solver* s, const double* psi_host);
 /* Run each step's launch sequences as HIP graphs (on = 1): the sequence from
  * H psi to the read of the step's energy and residual norm, and the one from
  * the preconditioner to the norms of the updated psi, each captured the
  * second time the same host decisions shape it (same Newton-Schulz step
  * count, Anderson state and buffers) and replayed from then on.  Steps with
- * Cholesky, a network trial or a restore, and profiled steps, run eagerly.
+ * an inverse from S itself, a network trial or a restore, and profiled steps,
+ * run eagerly.
  * Results are those of the eager launches.  No counterpart in the reference
  * (its steps are host loops). */
 int mgx_solver_set_graph(mgx_solver* s, int on);

@@ -1204,7 +1204,7 @@ int spd_inv_launch(mgx_ctx* ctx, int n, const double* S, double* X, double* info
 int spd_check(mgx_ctx* ctx, double info)
 {
     if (info == 0.) return MGX_OK;
-    return set_err(ctx, MGX_ENOTSPD, "ERROR in GramMatrix<MatrixType>::updateLS(): potrf info != 0");
+    return set_err(ctx, MGX_ENOTSPD, "matrix not positive definite (pivot " + std::to_string((int)info) + ")");
 }
 
 // spd_inv_launch with its check (waits for the stream)
@@ -1419,7 +1419,7 @@ int inverse_update_spec(mgx_ctx* ctx, int n, const double* Sv, const PairTiles& 
 // The checks inverse_update_pairs makes step by step, on the deltas of
 // inverse_update_spec: 0 = the steps were enough (*needed = the steps the
 // checked loop would have taken), 1 = they converge but more are needed,
-// -1 = they do not converge (Cholesky).  With final (the BF16 steps)
+// -1 = they do not converge (spd_inv).  With final (the BF16 steps)
 // deltas[nsteps] holds the measured error of the final X, and only a
 // measured delta below tol accepts.
 int ns_spec_check(const double* deltas, int nsteps, double tol, bool final, int* needed)

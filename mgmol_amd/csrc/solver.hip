@@ -143,8 +143,8 @@ struct mgx_solver
     int ns_pred = 2;  // Newton-Schulz steps taken without host checks (the last step's need)
     int ns_max_spec = 4;
     double ns_tol   = 1e-15;
-    int last_more   = 0;  // outcome of the last ns_spec_check (0 accepted, 1 continued, -1 Cholesky)
-    int64_t ns_continued = 0, ns_restarts = 0;  // checked continuations, Cholesky restarts of the refresh
+    int last_more   = 0;  // outcome of the last ns_spec_check (0 accepted, 1 continued, -1 diverged)
+    int64_t ns_continued = 0, ns_restarts = 0;  // checked continuations, restarts of the refresh from S
     int64_t gsize = 0;
     double* host = nullptr;  // pinned: [energy, norm]
     // HIP graphs of the step's launch sequences, by the host decisions that
@@ -214,7 +214,7 @@ int project(mgx_solver* s, int spec, bool bf16, int& tk)
 }
 
 // The launches of a step up to the host read of its scalars: H psi (with the
-// pending normalisation), S and H, S^-1 (symmetric sweeps, or spec
+// pending normalisation), S and H, S^-1 (from S, or by spec
 // Newton-Schulz steps whose deltas the host checks), theta, the energy, the
 // residual and its norm.  Changes no host state.
 int head_body(mgx_solver* s, bool pending, bool chol, int spec, bool bf16)
@@ -237,7 +237,7 @@ int head_body(mgx_solver* s, bool pending, bool chol, int spec, bool bf16)
     if ((rc = box_gram_h(ctx, s->bs, s->cfg.gram_prec, s->psi, s->hpsi, s->S, s->H, s->Sv, s->Hv))) return rc;
     prof_end(ctx, tk);
     tk = prof_begin(ctx, MGX_PROF_DENSE);
-    // S^-1: symmetric sweeps (GramMatrix::updateLS / computeInverse), or
+    // S^-1 from S (GramMatrix::updateLS / computeInverse), or
     // the Newton-Schulz refresh from the previous inverse
     if (chol)
     {
@@ -357,7 +357,7 @@ int tail_body(mgx_solver* s, bool use_cnn, bool restored, bool plain_step, doubl
 
 // The same for the Mehrstellen discretisation (FDtype = Mehrstellen): H psi
 // = -Lap_M psi + B V psi and B psi on the boxes, the Galerkin S, H and
-// B-matrix, S^-1 and B-matrix^-1 by symmetric sweeps (GramMatrix,
+// B-matrix, S^-1 and B-matrix^-1 (GramMatrix,
 // ProjectedMatricesMehrstellen::computeInvB,
 // src/ProjectedMatricesMehrstellen.cc:38-64), theta = B-matrix^-1 H
 // (updateTheta, .h:57-62), the band energy tr(HB S^-1) = tr(theta)
@@ -453,7 +453,7 @@ int step_body(mgx_solver* s, double tol, mgx_solver_stats_t* st, bool* done)
     const int n = s->n;
     const double ns_tol = s->ns_tol;
     const bool bf16     = s->cfg.inverse_mode == MGX_INV_NS_BF16;
-    // Cholesky on the first step (every step with MGX_INV_CHOL); else as
+    // S^-1 from S on the first step (every step with MGX_INV_CHOL); else as
     // many Newton-Schulz steps as the last refresh needed, unchecked, their
     // deltas checked with the energy and the residual norm below
     const bool mehr    = s->cfg.lap_type == MGX_LAP_MEHRSTELLEN;
@@ -470,7 +470,7 @@ int step_body(mgx_solver* s, double tol, mgx_solver_stats_t* st, bool* done)
                          && s->cfg.precond_start == MGX_START_ZERO;
     }
     if (mehr)
-        rc = head_mehr(s, pending);  // Cholesky of S and of the B-matrix every step
+        rc = head_mehr(s, pending);  // the inverses of S and of the B-matrix every step
     else if (chol)
         rc = head_body(s, pending, true, 0, bf16);  // the first step and restarts: never captured
     else
@@ -510,8 +510,8 @@ int step_body(mgx_solver* s, double tol, mgx_solver_stats_t* st, bool* done)
         else
         {
             // the unchecked steps were too few or did not converge: finish
-            // the inverse as inverse_update_pairs does (Cholesky when the
-            // steps diverged), then theta, the residual and its norm again
+            // the inverse as inverse_update_pairs does (from S when the steps
+            // diverged), then theta, the residual and its norm again
             tk = prof_begin(ctx, MGX_PROF_DENSE);
             int steps = 0;
             if (more < 0)

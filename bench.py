@@ -10,8 +10,8 @@ Paths, on identical inputs:
             products to 1e-15;
   mixed   : FP32 V-cycle (the reference's MGPRECONDTYPE), hi/lo-split S/H on
             FP32 MFMA with FP64 totals, S^-1 refreshed with FP64 Newton-Schulz
-            products (to 1e-10, the split S's own accuracy) and Cholesky in
-            FP64 where the refresh fails;
+            products (to 1e-10, the split S's own accuracy) and formed from S
+            in FP64 where the refresh fails;
   learned : mixed, with the trained BF16 CNN tried in place of the V-cycle
             (a plain preconditioned step, compared with the V-cycle step
             from the same state; the V-cycle takes over after a rejection);
@@ -21,7 +21,9 @@ Paths, on identical inputs:
 H psi, the residual and the energy are FP64 in all paths.
 value = seconds per converged solve of the mixed+learned path (lower is
 better), timed with kernel profiling off; the other paths' times, iteration
-counts and band-energy differences are reported beside it.
+counts and band-energy differences are reported beside it.  The printed line
+holds what fits a few kilobytes; --details FILE gets every group's and path's
+figures.
 
 Roofline: every kernel group the solver brackets with hipEvents (one
 profiled solve per path after the timed ones) carries its algorithmic bytes
@@ -68,7 +70,7 @@ PATHS = {
 }
 LABELS = {
     "plain": "plain FP64 (FP64 V-cycle, FP64 S/H, FP64 Newton-Schulz S^-1)",
-    "mixed": "mixed (FP32 V-cycle, hi/lo-split S/H, FP64 Newton-Schulz / Cholesky S^-1)",
+    "mixed": "mixed (FP32 V-cycle, hi/lo-split S/H, FP64 Newton-Schulz S^-1)",
     "learned": "mixed+learned (BF16 CNN preconditioner with the FP32 V-cycle as judge and fallback, "
                "hi/lo-split S/H, FP64 S^-1)",
     "ext16": "extension, not the specified precisions: FP16-storage V-cycle, hi/lo-split S/H, "
@@ -136,7 +138,8 @@ def run_mode(ctx, bs, cfg, mode, tol, maxit, steps, warmup, cnn, graph=True, nog
             t0 = time.perf_counter()
             st = s.run(tol, maxit)
             nograph.append(time.perf_counter() - t0)
-            log("[%s] solve without graphs %d: %d iterations, %.3f s" % (mode, k, st.iterations, nograph[-1]))
+            if k % 5 == 0 or k == nograph_steps - 1:
+                log("[%s] solve without graphs %d: %d iterations, %.3f s" % (mode, k, st.iterations, nograph[-1]))
         s.set_graph(graph)
     times, stats = [], None
     g0 = s.graph_stats()
@@ -145,9 +148,10 @@ def run_mode(ctx, bs, cfg, mode, tol, maxit, steps, warmup, cnn, graph=True, nog
         t0 = time.perf_counter()
         stats = s.run(tol, maxit)
         times.append(time.perf_counter() - t0)
-        log("[%s] solve %d: %d iterations, |R|=%.3e Ha, E=%.12f Ha, %.3f s (converged=%d, learned steps %d, "
-            "fallbacks %d)" % (mode, k, stats.iterations, stats.residual, stats.band_energy, times[-1],
-                               stats.converged, stats.learned_steps, stats.fallbacks))
+        if k % 5 == 0 or k == steps - 1:
+            log("[%s] solve %d: %d iterations, |R|=%.3e Ha, E=%.12f Ha, %.3f s (converged=%d, learned steps %d, "
+                "fallbacks %d)" % (mode, k, stats.iterations, stats.residual, stats.band_energy, times[-1],
+                                   stats.converged, stats.learned_steps, stats.fallbacks))
     g1 = s.graph_stats()
     # one more solve with the kernel groups timed (hipEvents on the engine's stream)
     s.reset()
@@ -277,6 +281,18 @@ def cpu_baseline(cfg, iters, mg_levels, budget_s=12.0):
                 cpus_available=cpu["cpus_available"])
 
 
+def brief(out):
+    """The printed line: of the tables, the figures that rank the groups and
+    compare the paths."""
+    o = {k: v for k, v in out.items() if k not in ("kernels", "phase_ms_per_solve", "autotune", "learned_training")}
+    o["paths"] = {m: {k: r[k] for k in ("seconds", "iterations", "energy", "residual", "converged", "learned_steps",
+                                        "fallbacks", "ns_restarts", "speedup_vs_plain", "energy_rel_diff_vs_plain")
+                      if k in r} for m, r in out["paths"].items()}
+    o["roofline_other"] = [{k: e.get(k) for k in ("group", "ms_per_solve", "bound", "achieved", "unit", "frac",
+                                                  "share_of_solve")} for e in out["roofline_other"]]
+    return o
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -289,6 +305,7 @@ def main():
     ap.add_argument("--modes", default="plain,mixed,learned,ext16")
     ap.add_argument("--weights", default=WEIGHTS)
     ap.add_argument("--no-cpu", action="store_true")
+    ap.add_argument("--details", help="write every figure (JSON) to this file")
     ap.add_argument("--no-graph", action="store_true", help="launch every kernel eagerly")
     args = ap.parse_args()
     if args.gpus != 1:
@@ -404,7 +421,10 @@ def main():
         cnn.close()
     bs.close()
     ctx.close()
-    print(json.dumps(out))
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(out, f, indent=1)
+    print(json.dumps(brief(out)))
 
 
 if __name__ == "__main__":

@@ -2030,6 +2030,9 @@ inline int64_t npoints(const mgx_grid_t& g) { return (int64_t)g.dim[0] * g.dim[1
 // level), and the first level that k_mg_coarse takes over (grids.size() if
 // none): the first one from level 1 whose points its threads hold and whose
 // arrays, with all coarser ones', fit the LDS.
+// That is so for any number of functions (blocks): three levels from 32^3 in
+// FP64, 1 function 59 us against 81 with every level by launches, 64 functions
+// 99 and 122, 1024 functions 959 and 1061; from 16^3, 3000 functions 501 and 630.
 constexpr size_t kMcLds = 150 * 1024;
 template <typename T>
 struct MgPacked

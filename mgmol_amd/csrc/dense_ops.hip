@@ -1153,7 +1153,7 @@ int chol_inv(mgx_ctx* ctx, int n, const double* S, double* L, double* Sinv)
 // own rows): W = Q L^-T, X - W W^T, and the column itself becomes W L^-1.  The
 // part not yet reached is so reduced as by a Cholesky factorisation; with the
 // block's inverse instead (X - Q A^-1 Q^T) it took errors of the order of
-// cond(A) and |I - S X| was 25 times (cond 1e6) to 3e4 times (1e13) the
+// cond(A) and |I - S X| was 25 times (cond 1e6) to 4e4 times (1e13) the
 // library's at n = 400.  Six launches a block.
 // info (device) receives 1 + the index of the first pivot that is not
 // positive, else 0.  n = 2048: 2.05 ms against the library's 7.3 ms;
